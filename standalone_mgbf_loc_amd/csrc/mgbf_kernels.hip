@@ -191,47 +191,20 @@ prolong2_kernel(const float* __restrict__ coarse, const float* addend, float* ou
 // next row needs two new fine rows. Rows and columns within S::EDGE of an
 // edge carry the folded mirror contributions and use the window tables.
 // ---------------------------------------------------------------------------
-// Edge tile of the restriction: window tables in x and y, one coarse point
-// at a time (only the tiles within two columns of an edge come here).
-template <int TI2>
-__device__ void restrict_edge_tile(const float* __restrict__ fine, float* __restrict__ coarse,
-                                   int kk, bool kvalid, int K, int nf, int mf, int I0, int J0,
-                                   int J1, const int* __restrict__ rxs,
-                                   const float* __restrict__ rxw, const int* __restrict__ rys,
-                                   const float* __restrict__ ryw) {
-    constexpr int WR = kRWidthDev;
-    const int nc = nf / 2;
-    const size_t frow = (size_t)nf * K;
-    for (int c = 0; c < TI2; ++c) {
-        const int I = I0 + c;
-        if (I >= nc) break;
-        const int xs = rxs[I];
-        for (int J = J0; J < J1; ++J) {
-            const int ys = rys[J];
-            float acc = 0.f;
-            for (int ty = 0; ty < WR; ++ty) {
-                const int jj = ys + ty < mf ? ys + ty : mf - 1;
-                const float wy = ys + ty < mf ? ryw[J * WR + ty] : 0.f;
-                const float* row = fine + kk + (size_t)jj * frow;
-                float a = 0.f;
-                for (int tx = 0; tx < WR; ++tx) {
-                    const int ii = xs + tx < nf ? xs + tx : nf - 1;
-                    const float wx = xs + tx < nf ? rxw[I * WR + tx] : 0.f;
-                    const float fv = row[(size_t)ii * K];
-                    a = __builtin_fmaf(wx, fv, a);
-                }
-                acc = __builtin_fmaf(wy, a, acc);
-            }
-            if (kvalid) coarse[kk + (size_t)K * ((size_t)I + (size_t)nc * J)] = acc;
-        }
-    }
-}
-
-template <int TI2, int TJ2, bool Q>
+// A wave whose columns lie within S::EDGE of a domain edge reads each coarse
+// column's own 8-column window with the weights of the x table (wave-uniform
+// scalar loads); everything else is the same for both, so an edge tile takes
+// about as long as an interior one: 256^2 x 64 in 18 us, 1440 x 960 x 65 and
+// its next two generations in 105 us each on average for the first two and
+// 27 us (162 us and 303, 203 and 172 us when an edge tile worked through one
+// coarse point at a time, 64 dependent loads each, in strips of 16 rows).
+// What bounds it is the latency of the two new fine rows of a coarse row.
+// The rows per wave tj2 are a launch parameter: launch_restrict.
+template <int TI2, bool Q>
 __global__ void __launch_bounds__(kBlock)
 restrict3_kernel(const float* __restrict__ fine, float* __restrict__ coarse, int K, int nf,
                  int mf, const int* __restrict__ rxs, const float* __restrict__ rxw,
-                 const int* __restrict__ rys, const float* __restrict__ ryw, int nkc, int ntile_i,
+                 const int* __restrict__ rys, const float* __restrict__ ryw, int tj2, int nkc, int ntile_i,
                  int nstrip, int nitems) {
     constexpr int WR = kRWidthDev;
     using S = Stencil<Q>;
@@ -252,19 +225,38 @@ restrict3_kernel(const float* __restrict__ fine, float* __restrict__ coarse, int
     const bool kvalid = k < K;
     const int kk = kvalid ? k : K - 1;
     const int nc = nf / 2, mc = mf / 2;
-    const int I0 = ti * TI2, J0 = js * TJ2;
-    const int J1 = J0 + TJ2 < mc ? J0 + TJ2 : mc;
-    if (!(I0 >= E && I0 + TI2 <= nc - E)) {
-        restrict_edge_tile<TI2>(fine, coarse, kk, kvalid, K, nf, mf, I0, J0, J1, rxs, rxw, rys, ryw);
-        return;
-    }
+    const int I0 = ti * TI2, J0 = js * tj2;
+    const int J1 = J0 + tj2 < mc ? J0 + tj2 : mc;
+    const bool xedge = !(I0 >= E && I0 + TI2 <= nc - E);
     const size_t frow = (size_t)nf * K;
     // interior columns: fine columns 2*I0+ROFF .. 2*I0+ROFF+NCF-1, addressed
     // as the row's buffer + lane k + wave-uniform column offset
-    const float* base = fine + (size_t)(2 * I0 + S::ROFF) * K;
+    const float* base = fine + (xedge ? (size_t)0 : (size_t)(2 * I0 + S::ROFF) * K);
     const int vk = kk * 4;
     auto xrow = [&](int fr, float* out) {
         const __amdgpu_buffer_rsrc_t rs = buf_rsrc(base + (size_t)fr * frow);
+        if (xedge) {
+            float v[TI2][WR];
+#pragma unroll
+            for (int c = 0; c < TI2; ++c) {
+                const int s0 = rxs[I0 + c < nc ? I0 + c : nc - 1];
+#pragma unroll
+                for (int t = 0; t < WR; ++t) v[c][t] = buf_ld(rs, vk, (s0 + t < nf ? s0 + t : nf - 1) * K * 4);
+            }
+#pragma unroll
+            for (int c = 0; c < TI2; ++c) {
+                const int I = I0 + c < nc ? I0 + c : nc - 1;
+                const int s0 = rxs[I];
+                float a = 0.f;
+#pragma unroll
+                for (int t = 0; t < WR; ++t) {
+                    const float w = s0 + t < nf ? rxw[I * WR + t] : 0.f;
+                    a = __builtin_fmaf(w, v[c][t], a);
+                }
+                out[c] = a;
+            }
+            return;
+        }
         float v[NCF];
 #pragma unroll
         for (int c = 0; c < NCF; ++c) v[c] = buf_ld(rs, vk, c * K * 4);
@@ -306,6 +298,7 @@ restrict3_kernel(const float* __restrict__ fine, float* __restrict__ coarse, int
             const int ys = rys[J];
 #pragma unroll
             for (int c = 0; c < TI2; ++c) acc[c] = 0.f;
+#pragma unroll
             for (int t = 0; t < WR; ++t) {
                 const int jj = ys + t < mf ? ys + t : mf - 1;
                 const float wy = ys + t < mf ? ryw[J * WR + t] : 0.f;
@@ -319,7 +312,8 @@ restrict3_kernel(const float* __restrict__ fine, float* __restrict__ coarse, int
         if (kvalid) {
             const __amdgpu_buffer_rsrc_t ro = buf_rsrc(coarse + (size_t)K * ((size_t)I0 + (size_t)nc * J));
 #pragma unroll
-            for (int c = 0; c < TI2; ++c) buf_st(acc[c], ro, vk, c * K * 4);
+            for (int c = 0; c < TI2; ++c)
+                if (I0 + c < nc) buf_st(acc[c], ro, vk, c * K * 4);
         }
     }
 }
@@ -440,20 +434,26 @@ hipError_t launch_ball3(const Ball3Args& a, hipStream_t st) {
 }
 
 hipError_t launch_restrict(const TransferArgs& a, hipStream_t st) {
-    constexpr int TI2 = 4, TJ2 = 16;
+    constexpr int TI2 = 4;
     const int nc = a.nf / 2, mc = a.mf / 2;
     const int ntile_i = (nc + TI2 - 1) / TI2;
-    const int nstrip = (mc + TJ2 - 1) / TJ2;
     const int nkc = (a.K + kWave - 1) / kWave;
+    // Coarse rows per wave: 16 read 38 fine rows (2.4 a row) where 4 read 14
+    // (3.5 a row), so shorter strips pay only while the launch leaves SIMDs
+    // without a wave to hide the loads of the others.
+    int tj2 = 16;
+    while (tj2 > 2 && (long long)ntile_i * nkc * ((mc + tj2 - 1) / tj2) < 8192) tj2 /= 2;
+    const int nstrip = (mc + tj2 - 1) / tj2;
     const long long nitems = (long long)ntile_i * nstrip * nkc;
+    if (nitems >= (1ll << 31)) return hipErrorInvalidValue;
     const unsigned nblocks = (unsigned)((nitems + kWavesPerBlock - 1) / kWavesPerBlock);
     if (a.quad)
-        hipLaunchKernelGGL((restrict3_kernel<TI2, TJ2, true>), dim3(nblocks), dim3(kBlock), 0, st,
-                           a.src, a.dst, a.K, a.nf, a.mf, a.xs, a.xw, a.ys, a.yw, nkc,
+        hipLaunchKernelGGL((restrict3_kernel<TI2, true>), dim3(nblocks), dim3(kBlock), 0, st,
+                           a.src, a.dst, a.K, a.nf, a.mf, a.xs, a.xw, a.ys, a.yw, tj2, nkc,
                            ntile_i, nstrip, (int)nitems);
     else
-        hipLaunchKernelGGL((restrict3_kernel<TI2, TJ2, false>), dim3(nblocks), dim3(kBlock), 0, st,
-                           a.src, a.dst, a.K, a.nf, a.mf, a.xs, a.xw, a.ys, a.yw, nkc,
+        hipLaunchKernelGGL((restrict3_kernel<TI2, false>), dim3(nblocks), dim3(kBlock), 0, st,
+                           a.src, a.dst, a.K, a.nf, a.mf, a.xs, a.xw, a.ys, a.yw, tj2, nkc,
                            ntile_i, nstrip, (int)nitems);
     return hipGetLastError();
 }
