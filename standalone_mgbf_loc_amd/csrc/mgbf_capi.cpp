@@ -139,7 +139,8 @@ struct mgbf_ctx {
     const float* wfield[mgbf::kMaxGen] = {};
     float wconst[mgbf::kMaxGen] = {};
     // per-point aspect tensors (mgbf_set_aspect): the weights of every
-    // point's taps over the (2H+1)^2 box; F^T is then a filter of its own
+    // point's taps over the (2H+1)^2 box, then the same of F^T, which is a
+    // filter of its own
     float* d_aw[mgbf::kMaxGen] = {};
     bool aniso[mgbf::kMaxGen] = {};
     // analysis <-> filter transfer: separable window tables (direct: filter ->
@@ -419,14 +420,17 @@ int radial(mgbf_ctx* c, int g, const float* in, float* out, const float* wfield,
                     (coarse || rout ? (double)c->gsize[g + 1] : 0.0)),
              g);
     if (c->aniso[g]) {
-        // per-point aspect tensors: F or F^T on its own, then the weighting;
-        // no epilogue rides in it
+        // per-point aspect tensors: F or F^T with the weighting; no transfer
+        // or band epilogue rides in it
         if (coarse || rout || band >= 0)
             return fail(MGBF_ERR_ARG, "internal: epilogue fused into a per-point aspect pass");
-        mgbf::AspectArgs aa{in, out, c->d_aw[g], c->K, c->nx[g], c->ny[g], c->s.H};
+        const float* aw = c->d_aw[g];
+        if (transpose) {
+            const size_t nb = 2 * (size_t)c->s.H + 1;
+            aw += (size_t)c->nx[g] * c->ny[g] * nb * nb;
+        }
+        mgbf::AspectArgs aa{in, out, aw, c->K, c->nx[g], c->ny[g], c->s.H, wfield, wconst};
         HIP_TRY(mgbf::launch_aspect(aa, transpose, st), "aspect filter launch");
-        if (wfield || wconst != 1.0f)
-            HIP_TRY(mgbf::launch_scale(out, out, wfield, wconst, 0, c->gsize[g], st), "scale launch");
         return MGBF_OK;
     }
     mgbf::RadialArgs a{};
@@ -1671,9 +1675,14 @@ int mgbf_set_aspect(mgbf_ctx* c, int gen, const double* pasp2) {
     std::string err;
     const int st = mgbf::aspect_weights(c->s.cfg, c->s.H, c->nx[g], c->ny[g], pasp2, w, &err);
     if (st != MGBF_OK) return fail(st, err);
-    if (!c->d_aw[g]) HIP_TRY(hipMalloc(&c->d_aw[g], sizeof(float) * w.size()), "hipMalloc(aspect weights)");
+    // the taps of F, and behind them the rows of the transposed matrix
+    if (!c->d_aw[g]) HIP_TRY(hipMalloc(&c->d_aw[g], 2 * sizeof(float) * w.size()), "hipMalloc(aspect weights)");
     HIP_TRY(hipMemcpy(c->d_aw[g], w.data(), sizeof(float) * w.size(), hipMemcpyHostToDevice),
             "aspect weights upload");
+    HIP_TRY(mgbf::launch_aspect_transpose(c->d_aw[g], c->d_aw[g] + w.size(), c->nx[g], c->ny[g], c->s.H, nullptr),
+            "aspect weights transposition");
+    // a later apply may run on a stream that does not wait for this one
+    HIP_TRY(hipStreamSynchronize(nullptr), "aspect weights transposition");
     c->aniso[g] = true;
     ++c->version;
     return MGBF_OK;

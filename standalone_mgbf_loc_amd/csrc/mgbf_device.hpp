@@ -85,6 +85,85 @@ __device__ __forceinline__ float lane_from_below(float v) {
                                                               0xf, true));
 }
 
+// acc += sum over g < N of (lane g of w in the lane's 16 lanes) * v[g], one
+// DPP row broadcast inside each FMA (the compiler keeps a broadcast and an FMA
+// apart, which doubles the instructions). The wait in front covers a value of
+// w that a vector instruction wrote just before: a DPP read needs two wait
+// states after it.
+#define MGBF_FMAC_BCAST(g, op) "v_fmac_f32_dpp %0, %1, %" #op " row_newbcast:" #g " row_mask:0xf bank_mask:0xf\n\t"
+template <int N>
+__device__ __forceinline__ void fmac_row(float& acc, float w, const float* v) {
+    if constexpr (N == 1)
+        asm("s_nop 1\n\t"
+            MGBF_FMAC_BCAST(0, 2)
+            : "+v"(acc)
+            : "v"(w), "v"(v[0]));
+    else if constexpr (N == 3)
+        asm("s_nop 1\n\t"
+            MGBF_FMAC_BCAST(0, 2) MGBF_FMAC_BCAST(1, 3) MGBF_FMAC_BCAST(2, 4)
+            : "+v"(acc)
+            : "v"(w), "v"(v[0]), "v"(v[1]), "v"(v[2]));
+    else if constexpr (N == 5)
+        asm("s_nop 1\n\t"
+            MGBF_FMAC_BCAST(0, 2) MGBF_FMAC_BCAST(1, 3) MGBF_FMAC_BCAST(2, 4) MGBF_FMAC_BCAST(3, 5)
+            MGBF_FMAC_BCAST(4, 6)
+            : "+v"(acc)
+            : "v"(w), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]));
+    else if constexpr (N == 7)
+        asm("s_nop 1\n\t"
+            MGBF_FMAC_BCAST(0, 2) MGBF_FMAC_BCAST(1, 3) MGBF_FMAC_BCAST(2, 4) MGBF_FMAC_BCAST(3, 5)
+            MGBF_FMAC_BCAST(4, 6) MGBF_FMAC_BCAST(5, 7) MGBF_FMAC_BCAST(6, 8)
+            : "+v"(acc)
+            : "v"(w), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]));
+    else if constexpr (N == 9)
+        asm("s_nop 1\n\t"
+            MGBF_FMAC_BCAST(0, 2) MGBF_FMAC_BCAST(1, 3) MGBF_FMAC_BCAST(2, 4) MGBF_FMAC_BCAST(3, 5)
+            MGBF_FMAC_BCAST(4, 6) MGBF_FMAC_BCAST(5, 7) MGBF_FMAC_BCAST(6, 8) MGBF_FMAC_BCAST(7, 9)
+            MGBF_FMAC_BCAST(8, 10)
+            : "+v"(acc)
+            : "v"(w), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]),
+              "v"(v[8]));
+    else if constexpr (N == 11)
+        asm("s_nop 1\n\t"
+            MGBF_FMAC_BCAST(0, 2) MGBF_FMAC_BCAST(1, 3) MGBF_FMAC_BCAST(2, 4) MGBF_FMAC_BCAST(3, 5)
+            MGBF_FMAC_BCAST(4, 6) MGBF_FMAC_BCAST(5, 7) MGBF_FMAC_BCAST(6, 8) MGBF_FMAC_BCAST(7, 9)
+            MGBF_FMAC_BCAST(8, 10) MGBF_FMAC_BCAST(9, 11) MGBF_FMAC_BCAST(10, 12)
+            : "+v"(acc)
+            : "v"(w), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]),
+              "v"(v[8]), "v"(v[9]), "v"(v[10]));
+    else if constexpr (N == 13)
+        asm("s_nop 1\n\t"
+            MGBF_FMAC_BCAST(0, 2) MGBF_FMAC_BCAST(1, 3) MGBF_FMAC_BCAST(2, 4) MGBF_FMAC_BCAST(3, 5)
+            MGBF_FMAC_BCAST(4, 6) MGBF_FMAC_BCAST(5, 7) MGBF_FMAC_BCAST(6, 8) MGBF_FMAC_BCAST(7, 9)
+            MGBF_FMAC_BCAST(8, 10) MGBF_FMAC_BCAST(9, 11) MGBF_FMAC_BCAST(10, 12) MGBF_FMAC_BCAST(11, 13)
+            MGBF_FMAC_BCAST(12, 14)
+            : "+v"(acc)
+            : "v"(w), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]),
+              "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]));
+    else if constexpr (N == 15)
+        asm("s_nop 1\n\t"
+            MGBF_FMAC_BCAST(0, 2) MGBF_FMAC_BCAST(1, 3) MGBF_FMAC_BCAST(2, 4) MGBF_FMAC_BCAST(3, 5)
+            MGBF_FMAC_BCAST(4, 6) MGBF_FMAC_BCAST(5, 7) MGBF_FMAC_BCAST(6, 8) MGBF_FMAC_BCAST(7, 9)
+            MGBF_FMAC_BCAST(8, 10) MGBF_FMAC_BCAST(9, 11) MGBF_FMAC_BCAST(10, 12) MGBF_FMAC_BCAST(11, 13)
+            MGBF_FMAC_BCAST(12, 14) MGBF_FMAC_BCAST(13, 15) MGBF_FMAC_BCAST(14, 16)
+            : "+v"(acc)
+            : "v"(w), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]),
+              "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]), "v"(v[13]), "v"(v[14]));
+    else if constexpr (N == 16)
+        asm("s_nop 1\n\t"
+            MGBF_FMAC_BCAST(0, 2) MGBF_FMAC_BCAST(1, 3) MGBF_FMAC_BCAST(2, 4) MGBF_FMAC_BCAST(3, 5)
+            MGBF_FMAC_BCAST(4, 6) MGBF_FMAC_BCAST(5, 7) MGBF_FMAC_BCAST(6, 8) MGBF_FMAC_BCAST(7, 9)
+            MGBF_FMAC_BCAST(8, 10) MGBF_FMAC_BCAST(9, 11) MGBF_FMAC_BCAST(10, 12) MGBF_FMAC_BCAST(11, 13)
+            MGBF_FMAC_BCAST(12, 14) MGBF_FMAC_BCAST(13, 15) MGBF_FMAC_BCAST(14, 16) MGBF_FMAC_BCAST(15, 17)
+            : "+v"(acc)
+            : "v"(w), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "v"(v[4]), "v"(v[5]), "v"(v[6]), "v"(v[7]),
+              "v"(v[8]), "v"(v[9]), "v"(v[10]), "v"(v[11]), "v"(v[12]), "v"(v[13]), "v"(v[14]),
+              "v"(v[15]));
+    else
+        static_assert(N < 0, "a width that is not built");
+}
+#undef MGBF_FMAC_BCAST
+
 // Interpolation constants of the offset grids (def_offset_coef): fine index
 // 2u (even, 0-based) reads coarse u-2..u+1 with kQc, fine 2u+1 reads coarse
 // u-1..u+2 with kPc.

@@ -880,77 +880,228 @@ hipError_t launch_ball(const BallArgs& a, hipStream_t st) {
 
 // The radial filter of a generation whose aspect tensor varies per point
 // (vrbeta2 / vrbeta2T with el(:,:,ix,iy) and ss(ix,iy), jp_pbfil.f90:
-// 888-928, 1011-1050). Point p = i + n j carries the weights of its taps
-// over the box |gx|, |gy| <= H, w[p][t] with t = (gy+H)(2H+1) + gx+H
-// (ss included, zero off its ellipse). One wave per point and 64 k:
-//   F   (T = false): out(p) = sum_t w[p][t] in(mirror(p + g_t)), the gather
-//                    of vrbeta2 over the mirrored halo of boco_2d;
-//   F^T (T = true):  the scatter of vrbeta2T followed by the fold of
-//                    bocoT_2d, as a gather: out(q) = sum over the mirror
-//                    preimages e of q (per axis q, -1-q within H of the low
-//                    edge, 2n-1-q within H of the high one) and the taps t
-//                    whose source s = e - g_t lies in the domain, of
-//                    w[s][t] in(s).
+// 888-928, 1011-1050) as a gather: point p = i + n j carries its weights over
+// the box |gx|, |gy| <= H, w[p][t] with t = (gy+H)(2H+1) + gx+H.
+//   F   (T = false): out(p) = sum_t w[p][t] in(mirror(p + g_t)), the gather of
+//                    vrbeta2 over the mirrored halo of boco_2d (ss included,
+//                    zero off the point's ellipse);
+//   F^T (T = true):  out(p) = sum_t w[p][t] in(p + g_t) over the points of the
+//                    domain, with the rows of the transposed matrix (the
+//                    scatter of vrbeta2T and the fold of bocoT_2d, collected
+//                    per output point when the tensors are set; zero where
+//                    p + g_t lies outside).
+//
+// A wave computes TI x TJ outputs for its 64 k: each input row of the tile's
+// halo enters the TJ output rows with every output's own weights. A row of an
+// output's weights is one load that puts weight gx into lane gx of every 16
+// lanes (two loads from half-width 8 on), and the FMAs take it from there by
+// a DPP row broadcast, so a weight costs no instruction of its own. Inputs and
+// weights of two rows are in flight while a third is combined: what bounds it
+// is the (2H+1)^2 FMAs of an output (a third of their rate at 256 x 256 x 64,
+// H = 6: 36 us for F and for F^T), and on a small grid the latency of the
+// rows (20 us at 64 x 64 x 64). One tap at a time, behind a scalar load, a
+// vector load and a branch on the weight, took 438 us (F) and 746 us (F^T);
+// the weights as scalar operands 80 us, waiting on the scalar loads.
+// Zero weights are multiplied like the others, which differs from leaving
+// the tap out only where an input is infinite or NaN: an output of the tile
+// that is not finite sends the wave through aspect_point, which leaves them
+// out.
+//
+// One output point by its taps one after the other, zero weights left out.
 template <bool T>
-__global__ void __launch_bounds__(kBlock) aspect_kernel(AspectArgs a, int nkc, long long nitems) {
-    const long long item = __builtin_amdgcn_readfirstlane(
-        (int)((long long)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6)));
-    if (item >= nitems) return;
-    const int kc = (int)(item % nkc);
-    const long long pt = item / nkc;
-    const int i = (int)(pt % a.n), j = (int)(pt / a.n);
-    const int k = kc * kWave + (threadIdx.x & (kWave - 1));
-    const bool kv = k < a.K;
-    const int kk = kv ? k : a.K - 1;
-    const int H = a.H, NB = 2 * H + 1, nt = NB * NB, n = a.n, m = a.m;
+__device__ float aspect_point(const AspectArgs& a, int i, int j, int kk) {
+    const int H = a.H, NB = 2 * H + 1, n = a.n, m = a.m;
     const size_t K = (size_t)a.K;
+    const float* wp = a.w + ((size_t)i + (size_t)n * j) * NB * NB;
     float acc = 0.f;
-    if (!T) {
-        const float* wp = a.w + (size_t)(i + (size_t)n * j) * nt;
-        for (int gy = -H; gy <= H; ++gy) {
-            const int jj = mirror_half(j + gy, m);
-            for (int gx = -H; gx <= H; ++gx) {
-                const float wv = wp[(gy + H) * NB + gx + H];
-                if (wv != 0.f)
-                    acc = __builtin_fmaf(wv, a.in[kk + K * ((size_t)mirror_half(i + gx, n) + (size_t)n * jj)], acc);
+    for (int gy = -H; gy <= H; ++gy)
+        for (int gx = -H; gx <= H; ++gx) {
+            const float wv = wp[(gy + H) * NB + gx + H];
+            if (wv == 0.f) continue;
+            // F^T has no weight on a point outside the domain
+            const int ii = T ? i + gx : mirror_half(i + gx, n), jj = T ? j + gy : mirror_half(j + gy, m);
+            acc = __builtin_fmaf(wv, a.in[kk + K * ((size_t)ii + (size_t)n * jj)], acc);
+        }
+    return acc;
+}
+
+template <int H, bool T>
+__global__ void __launch_bounds__(kBlock) aspect_kernel(AspectArgs a, int nkc, int ntile_i, int nitems) {
+    constexpr int TI = 4, TJ = 4, NB = 2 * H + 1, NT = NB * NB, NC = TI + 2 * H;
+    const int item = (int)xcd_block(blockIdx.x, gridDim.x) * kWavesPerBlock +
+                     __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (item >= nitems) return;
+    const int kc = item % nkc;
+    const int rest = item / nkc;
+    const int i0 = (rest % ntile_i) * TI, j0 = (rest / ntile_i) * TJ;
+    const int k = kc * kWave + (threadIdx.x & (kWave - 1));
+    const int K = a.K, n = a.n, m = a.m;
+    const bool kvalid = k < K;
+    const int vk = (kvalid ? k : K - 1) * 4;
+    const size_t rowstride = (size_t)n * K;
+    // a point outside the domain: its mirror image for F, any point for F^T
+    // (its weight is zero)
+    auto at = [](int q, int len) { return T ? (q < 0 ? 0 : (q < len ? q : len - 1)) : mirror_half(q, len); };
+    int voff[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) voff[c] = vk + at(i0 - H + c, n) * K * 4;
+    constexpr int NW = NB > 16 ? 2 : 1;
+    int wl[NW];   // this lane's weight of a row of weights, in bytes
+#pragma unroll
+    for (int e = 0; e < NW; ++e) {
+        const int gx = (threadIdx.x & 15) + 16 * e;
+        wl[e] = (gx < NB ? gx : NB - 1) * 4;
+    }
+    float acc[TJ][TI];
+#pragma unroll
+    for (int q = 0; q < TJ; ++q)
+#pragma unroll
+        for (int t = 0; t < TI; ++t) acc[q][t] = 0.f;
+    struct Row {
+        float v[NC];
+        float w[TJ][TI][NW];
+    };
+    auto used = [&](int r, int q) {   // does input row r enter output row j0 + q?
+        const int gy = r - (j0 + q);
+        return j0 + q < m && gy >= -H && gy <= H;
+    };
+    auto load = [&](int r, Row& d) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rs = buf_rsrc(a.in + (size_t)at(r, m) * rowstride);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) d.v[c] = buf_ld(rs, voff[c], 0);
+#pragma unroll
+        for (int q = 0; q < TJ; ++q) {
+            if (!used(r, q)) continue;
+            const __amdgpu_buffer_rsrc_t rw =
+                buf_rsrc(a.w + ((size_t)i0 + (size_t)n * (j0 + q)) * NT + (r - (j0 + q) + H) * NB);
+            // a column past the domain takes the last one's weights; its output is dropped
+#pragma unroll
+            for (int t = 0; t < TI; ++t)
+#pragma unroll
+                for (int e = 0; e < NW; ++e)
+                    d.w[q][t][e] = buf_ld(rw, wl[e], (i0 + t < n ? t : n - 1 - i0) * NT * 4);
+        }
+    };
+    auto combine = [&](int r, const Row& d) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < TJ; ++q) {
+            if (!used(r, q)) continue;
+#pragma unroll
+            for (int t = 0; t < TI; ++t) {
+                fmac_row<(NB < 16 ? NB : 16)>(acc[q][t], d.w[q][t][0], d.v + t);
+                if constexpr (NB > 16) fmac_row<NB - 16>(acc[q][t], d.w[q][t][1], d.v + t + 16);
             }
         }
-    } else {
-        int ex[3], ey[3], nx = 0, ny = 0;
-        ex[nx++] = i;
-        if (i <= H - 1) ex[nx++] = -1 - i;
-        if (i >= n - H) ex[nx++] = 2 * n - 1 - i;
-        ey[ny++] = j;
-        if (j <= H - 1) ey[ny++] = -1 - j;
-        if (j >= m - H) ey[ny++] = 2 * m - 1 - j;
-        for (int b = 0; b < ny; ++b)
-            for (int gy = -H; gy <= H; ++gy) {
-                const int sy = ey[b] - gy;
-                if (sy < 0 || sy >= m) continue;
-                for (int c = 0; c < nx; ++c)
-                    for (int gx = -H; gx <= H; ++gx) {
-                        const int sx = ex[c] - gx;
-                        if (sx < 0 || sx >= n) continue;
-                        const size_t sp = (size_t)sx + (size_t)n * sy;
-                        const float wv = a.w[sp * nt + (gy + H) * NB + gx + H];
-                        if (wv != 0.f) acc = __builtin_fmaf(wv, a.in[kk + K * sp], acc);
-                    }
+    };
+    static_assert((TJ + 2 * H) % 2 == 0, "rows come in pairs");
+    Row A, B;
+    load(j0 - H, A);
+    load(j0 - H + 1, B);
+    for (int r = j0 - H; r < j0 + TJ + H; r += 2) {
+        combine(r, A);
+        if (r + 2 < j0 + TJ + H) load(r + 2, A);
+        combine(r + 1, B);
+        if (r + 2 < j0 + TJ + H) load(r + 3, B);
+    }
+    bool odd = false;
+#pragma unroll
+    for (int q = 0; q < TJ; ++q)
+#pragma unroll
+        for (int t = 0; t < TI; ++t) odd = odd || !(__builtin_fabsf(acc[q][t]) < __builtin_inff());
+    if (__any(odd)) {
+        for (int q = 0; q < TJ; ++q)
+            for (int t = 0; t < TI; ++t)
+                if (j0 + q < m && i0 + t < n) {
+                    const float x = aspect_point<T>(a, i0 + t, j0 + q, vk / 4);
+#pragma unroll
+                    for (int e = 0; e < TJ * TI; ++e)
+                        if (e == q * TI + t) acc[e / TI][e % TI] = x;
+                }
+    }
+    if (!kvalid) return;
+#pragma unroll
+    for (int q = 0; q < TJ; ++q) {
+        const int j = j0 + q;
+        if (j >= m) break;
+        const size_t off = (size_t)j * rowstride + (size_t)i0 * K;
+        const __amdgpu_buffer_rsrc_t ro = buf_rsrc(a.out + off);
+        const __amdgpu_buffer_rsrc_t rw = buf_rsrc((a.wfield ? a.wfield : a.out) + off);
+#pragma unroll
+        for (int t = 0; t < TI; ++t)
+            if (i0 + t < n) {
+                const float s = a.wfield ? buf_ld(rw, vk, t * K * 4) : a.wconst;
+                buf_st(s * acc[q][t], ro, vk, t * K * 4);
             }
     }
-    if (kv) a.out[k + K * ((size_t)i + (size_t)n * j)] = acc;
+}
+
+// The rows of the transposed matrix from those of F: point p takes the weight
+// of every tap of p + g that reaches p, directly or through a mirror image of
+// p (the box holds all of them: folding moves a point towards the tap's
+// origin). One thread per weight.
+__global__ void __launch_bounds__(kBlock) aspect_transpose_kernel(const float* __restrict__ w, float* __restrict__ wt,
+                                                                int n, int m, int H, long long count) {
+    const long long e = (long long)blockIdx.x * kBlock + threadIdx.x;
+    if (e >= count) return;
+    const int NB = 2 * H + 1, nt = NB * NB;
+    const int t = (int)(e % nt);
+    const long long p = e / nt;
+    const int i = (int)(p % n), j = (int)(p / n);
+    const int sx = i + t % NB - H, sy = j + t / NB - H;
+    float acc = 0.f;
+    if (sx >= 0 && sx < n && sy >= 0 && sy < m) {
+        const float* ws = w + ((size_t)sx + (size_t)n * sy) * nt;
+        for (int b = 0; b < 3; ++b) {
+            const int gy = (b == 0 ? j : (b == 1 ? -1 - j : 2 * m - 1 - j)) - sy;
+            if (gy < -H || gy > H) continue;
+            for (int c = 0; c < 3; ++c) {
+                const int gx = (c == 0 ? i : (c == 1 ? -1 - i : 2 * n - 1 - i)) - sx;
+                if (gx >= -H && gx <= H) acc += ws[(gy + H) * NB + gx + H];
+            }
+        }
+    }
+    wt[e] = acc;
+}
+
+hipError_t launch_aspect_transpose(const float* w, float* wt, int n, int m, int H, hipStream_t st) {
+    const long long count = (long long)n * m * (2 * H + 1) * (2 * H + 1);
+    const long long nblocks = (count + kBlock - 1) / kBlock;
+    if (H < 1 || n < H || m < H || nblocks >= (1ll << 31)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(aspect_transpose_kernel, dim3((unsigned)nblocks), dim3(kBlock), 0, st, w, wt, n, m, H, count);
+    return hipGetLastError();
+}
+
+template <int H>
+hipError_t launch_aspect_h(const AspectArgs& a, bool transpose, hipStream_t st) {
+    const int nkc = (a.K + kWave - 1) / kWave, ntile_i = (a.n + 3) / 4, ntile_j = (a.m + 3) / 4;
+    const long long nitems = (long long)nkc * ntile_i * ntile_j;
+    const long long nblocks = (nitems + kWavesPerBlock - 1) / kWavesPerBlock;
+    // 32-bit offsets inside a row
+    if (nitems >= (1ll << 31) || (long long)(a.n + 16) * a.K * 4 >= (1ll << 31)) return hipErrorInvalidValue;
+    if (transpose)
+        hipLaunchKernelGGL((aspect_kernel<H, true>), dim3((unsigned)nblocks), dim3(kBlock), 0, st, a, nkc, ntile_i,
+                           (int)nitems);
+    else
+        hipLaunchKernelGGL((aspect_kernel<H, false>), dim3((unsigned)nblocks), dim3(kBlock), 0, st, a, nkc, ntile_i,
+                           (int)nitems);
+    return hipGetLastError();
 }
 
 hipError_t launch_aspect(const AspectArgs& a, bool transpose, hipStream_t st) {
     if (a.H < 1 || a.n < a.H || a.m < a.H || a.K < 1) return hipErrorInvalidValue;
-    const int nkc = (a.K + kWave - 1) / kWave;
-    const long long nitems = (long long)nkc * a.n * a.m;
-    const long long nblocks = (nitems + kWavesPerBlock - 1) / kWavesPerBlock;
-    if (nitems >= (1ll << 31)) return hipErrorInvalidValue;
-    if (transpose)
-        hipLaunchKernelGGL(aspect_kernel<true>, dim3((unsigned)nblocks), dim3(kBlock), 0, st, a, nkc, nitems);
-    else
-        hipLaunchKernelGGL(aspect_kernel<false>, dim3((unsigned)nblocks), dim3(kBlock), 0, st, a, nkc, nitems);
-    return hipGetLastError();
+    switch (a.H) {
+        case 1: return launch_aspect_h<1>(a, transpose, st);
+        case 2: return launch_aspect_h<2>(a, transpose, st);
+        case 3: return launch_aspect_h<3>(a, transpose, st);
+        case 4: return launch_aspect_h<4>(a, transpose, st);
+        case 5: return launch_aspect_h<5>(a, transpose, st);
+        case 6: return launch_aspect_h<6>(a, transpose, st);
+        case 7: return launch_aspect_h<7>(a, transpose, st);
+        case 8: return launch_aspect_h<8>(a, transpose, st);
+        case 9: return launch_aspect_h<9>(a, transpose, st);
+        case 10: return launch_aspect_h<10>(a, transpose, st);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 hipError_t launch_xfer2d(const XferArgs& a, hipStream_t st) {

@@ -140,14 +140,19 @@ struct VBandArgs {
 
 // The radial filter of a generation with a per-point aspect tensor field:
 // w holds, per point p = i + n j, the weights of the (2H+1)^2 offsets
-// |gx|, |gy| <= H (t = (gy+H)(2H+1) + gx+H), zero off the point's ellipse.
+// |gx|, |gy| <= H (t = (gy+H)(2H+1) + gx+H): the point's own taps for F,
+// its row of the transposed matrix for F^T.
 struct AspectArgs {
     const float* in;
     float* out;
     const float* w;
     int K, n, m, H;
+    const float* wfield;  // per-point scale of the output, or nullptr
+    float wconst;         // constant scale when wfield is nullptr
 };
 hipError_t launch_aspect(const AspectArgs& a, bool transpose, hipStream_t st);
+// wt = the rows of the transposed matrix, from the taps w of F
+hipError_t launch_aspect_transpose(const float* w, float* wt, int n, int m, int H, hipStream_t st);
 
 hipError_t launch_radial(const RadialArgs& a, hipStream_t st);
 hipError_t launch_vband(const VBandArgs& a, hipStream_t st);
