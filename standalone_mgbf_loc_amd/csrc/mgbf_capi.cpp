@@ -533,19 +533,30 @@ int restrict_chain(mgbf_ctx* c, const float* u1, float* U, hipStream_t st) {
     return MGBF_OK;
 }
 
+// Which weights ride in a pass: none, A_g, or A_g^{1/2} where it is a
+// constant (a scale of the pass's output like A_g; the square root of a
+// per-point field stays a scale pass of its own).
+enum class Weight { None, A, SqrtConst };
+
+// The constant a pass of generation g is scaled by under w, per-point fields aside.
+float pass_const(const mgbf_ctx* c, int g, Weight w) {
+    if (w == Weight::A) return c->wconst[g];
+    return w == Weight::SqrtConst && !c->wfield[g] ? std::sqrt(c->wconst[g]) : 1.0f;
+}
+
 // Down-sweep: the first radial pass of every filtered generation,
-// T_g = A_g F u_g (A_g = 1 unless `weighted`), written at T + goff[g], and
+// T_g = A_g F u_g (or with the weights of `weight`), written at T + goff[g], and
 // the restriction u_{g+1} = R u_g into U + goff[g+1]. The restriction rides
 // in the radial pass where the tiles allow (fusion level 3), else it runs on
 // its own first. u_1 is read from u1.
-int down_sweep(mgbf_ctx* c, const float* u1, float* U, float* T, bool weighted, hipStream_t st) {
+int down_sweep(mgbf_ctx* c, const float* u1, float* U, float* T, Weight weight, hipStream_t st) {
     for (int g = 0; g < c->gm; ++g) {
         const float* ug = g == 0 ? u1 : U + c->goff[g];
         const bool last = g + 1 >= c->gm;
         const bool filt = g > 0 || c->filt_g1;
         float* next = last ? nullptr : U + c->goff[g + 1];
-        const float* wf = weighted ? c->wfield[g] : nullptr;
-        const float wc = weighted ? c->wconst[g] : 1.0f;
+        const float* wf = weight == Weight::A ? c->wfield[g] : nullptr;
+        const float wc = pass_const(c, g, weight);
         if (filt && !last && c->fuse >= 3 && !c->aniso[g] && fused_ok(c, g, c->tile_tj[g][3], c->s.H)) {
             CALL(radial(c, g, ug, T + c->goff[g], wf, wc, st, MGBF_T_HFILTT, nullptr, -1, next));
             continue;
@@ -559,7 +570,8 @@ int down_sweep(mgbf_ctx* c, const float* u1, float* U, float* T, bool weighted, 
 // Up-sweep from the coarsest generation: for g = gm..1 (1-based)
 //   s_g = F in_g + P s_{g+1},  in_1 = in1, in_g = inb + goff[g] (g >= 2)
 // (in_g = T_g after a down-sweep for W A W^T; the control vector's v_g for W,
-// scaled by A_g^{1/2} first when sqrt_w). s_g is written into U. The last
+// with A_g^{1/2} v_g when sqrt_w: a constant scales F v_g in the pass, a
+// field scales v_g first). s_g is written into U. The last
 // pass writes y = band(s_1) directly when the vertical band fuses (or there
 // is none), else s_1 goes to U0 and a separate vertical pass follows. An
 // unfiltered generation 1 gives s_1 = u1 + P s_2.
@@ -583,12 +595,13 @@ int upsweep(mgbf_ctx* c, const float* in1, const float* inb, const float* u1, fl
             else if (u1 != s1) HIP_TRY(mgbf::launch_copy(u1, s1, c->gsize[0], st), "copy launch");
             return band >= 0 ? vertical(c, U, y, band, st) : MGBF_OK;
         }
-        if (sqrt_w) {
+        if (sqrt_w && c->wfield[g]) {
             HIP_TRY(mgbf::launch_scale(src, T, c->wfield[g], c->wconst[g], 1, c->gsize[g], st),
                     "scale launch");
             src = T;
         }
-        CALL(radial(c, g, src, dst, nullptr, 1.0f, st, MGBF_T_HFILT, pro, fb));
+        const float wc = pass_const(c, g, sqrt_w ? Weight::SqrtConst : Weight::None);
+        CALL(radial(c, g, src, dst, nullptr, wc, st, MGBF_T_HFILT, pro, fb));
         if (coarse && !pro) CALL(prolong_g(c, g, coarse, dst, dst, st));
     }
     if (band >= 0 && !fuse) return vertical(c, U, y, band, st);
@@ -600,7 +613,7 @@ int upsweep(mgbf_ctx* c, const float* in1, const float* inb, const float* u1, fl
 // vertical filter, B = Vf H Vf^T = (Vf Vf^T) H; one banded vertical pass,
 // fused into the last radial pass when possible.
 int apply_wawt_commuted(mgbf_ctx* c, const float* x, float* y, hipStream_t st) {
-    CALL(down_sweep(c, x, c->ws_u, c->ws_t, true, st));
+    CALL(down_sweep(c, x, c->ws_u, c->ws_t, Weight::A, st));
     return upsweep(c, c->ws_t, c->ws_t, x, y, c->nfilt ? BAND_VVT : -1, false, st);
 }
 
@@ -610,20 +623,20 @@ int apply_wawt(mgbf_ctx* c, const float* x, float* y, hipStream_t st) {
     if (!fields && c->commute) return apply_wawt_commuted(c, x, y, st);
     float* U = c->ws_u;
     CALL(vertical(c, x, U, BAND_VFT, st));
-    CALL(down_sweep(c, U, U, c->ws_t, true, st));
+    CALL(down_sweep(c, U, U, c->ws_t, Weight::A, st));
     return upsweep(c, c->ws_t, c->ws_t, U, y, c->nfilt ? c->vf_last : -1, false, st);
 }
 
 int apply_wt(mgbf_ctx* c, const float* x, float* v, bool sqrt_weights, hipStream_t st) {
     float* U = c->ws_u;
     CALL(vertical(c, x, U, BAND_VFT, st));
-    CALL(down_sweep(c, U, U, v, false, st));
+    CALL(down_sweep(c, U, U, v, sqrt_weights ? Weight::SqrtConst : Weight::None, st));
     for (int g = 0; g < c->gm; ++g) {
         if (g == 0 && !c->filt_g1) {
             HIP_TRY(mgbf::launch_copy(U, v, c->gsize[0], st), "copy launch");
             continue;
         }
-        if (sqrt_weights)
+        if (sqrt_weights && c->wfield[g])
             HIP_TRY(mgbf::launch_scale(v + c->goff[g], v + c->goff[g], c->wfield[g], c->wconst[g], 1,
                                        c->gsize[g], st),
                     "scale launch");
