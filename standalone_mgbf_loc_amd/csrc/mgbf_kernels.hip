@@ -115,6 +115,121 @@ vband_kernel(const float* __restrict__ in, float* __restrict__ out,
     }
 }
 
+// The same operator where every column is filtered but no column fits the
+// block (lm = 65, 127). A block takes 64 whole columns, lane l of its 4 waves
+// column l, each wave a quarter of the levels: the level, and with it the band
+// row, is the same in all lanes (scalar coefficients, read from memory only
+// next to the column ends). The columns' contiguous span passes LDS in 16-byte
+// pieces; a wave walks down its levels with the window in registers and leaves
+// the results in place, past a copy of the HB levels below its quarter, which
+// the next wave overwrites. An element passes LDS 4 times where the block
+// above reads it 2 HB + 1 times and finds its level by two divisions. A pitch
+// of lm keeps the lanes in different banks for odd lm, in pairs for
+// lm = 2 mod 4. HBM is the bound, and LDS (lm x 256 bytes a block) limits the
+// blocks that hide its latency: 1440 x 960 x 65 at HB = 6, 0.72 GB, in 139 us
+// against 278 with the block above; 1024 x 1024 x 127 at HB = 3, 1.07 GB, in
+// 193 against 268 (one wave a column block, without the quarters, took 396).
+// ---------------------------------------------------------------------------
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+constexpr int kVColMaxHB = 8;     // hz <= 4; wider windows take the block above
+constexpr int kVColMaxLm = 128;   // 32 KB of columns: 4 blocks, 16 waves a CU
+constexpr int kVColWaves = kBlock / kWave;
+constexpr int kVColStep = 8;      // levels between shifts of the window
+
+template <int HB, bool VEC>
+__global__ void __launch_bounds__(kBlock)
+vcol_kernel(const float* __restrict__ in, float* __restrict__ out, const float* __restrict__ band, VBandW wint,
+            int ilo, int ihi, int lm, long long ncol) {
+    constexpr int NB = 2 * HB + 1;
+    extern __shared__ __align__(16) float s_mem[];
+    float* const s_halo = s_mem;                                // [wave][HB][64]
+    float* const s_col = s_mem + kVColWaves * HB * kWave;       // [64][lm]
+    const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const long long c0 = (long long)blockIdx.x * kWave;
+    const int cols = (int)(ncol - c0 < kWave ? ncol - c0 : kWave);
+    const int span = cols * lm;
+    const float* src = in + c0 * lm;
+    float* dst = out + c0 * lm;
+    // 8 loads in flight; those past the span's last 16 bytes read nothing
+    const int n4 = span >> 2;
+    constexpr int kStep = 8;
+    if constexpr (VEC) {
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src), (short)0, n4 * 16, 0x00020000);
+        for (int e0 = 0; e0 < n4; e0 += kStep * kBlock) {
+            u4 v[kStep];
+#pragma unroll
+            for (int q = 0; q < kStep; ++q)
+                v[q] = __builtin_amdgcn_raw_buffer_load_b128(rs, (e0 + q * kBlock + tid) * 16, 0, 0);
+#pragma unroll
+            for (int q = 0; q < kStep; ++q) {
+                const int e = e0 + q * kBlock + tid;
+                if (e < n4) reinterpret_cast<f4*>(s_col)[e] = __builtin_bit_cast(f4, v[q]);
+            }
+        }
+        if (4 * n4 + tid < span) s_col[4 * n4 + tid] = src[4 * n4 + tid];
+    } else {
+        for (int e = tid; e < span; e += kBlock) s_col[e] = src[e];
+    }
+    __syncthreads();
+    // levels l0 .. l1 - 1 are this wave's; lanes past the last column work on
+    // their unused places
+    const int q4 = (lm + kVColWaves - 1) / kVColWaves;
+    const int l0 = wave * q4 < lm ? wave * q4 : lm, l1 = l0 + q4 < lm ? l0 + q4 : lm;
+    float* const col = s_col + lane * lm;
+    float* const halo = s_halo + wave * HB * kWave + lane;
+    // w[t]: level L0 + t - HB; levels outside the column read as zero
+    float w[2 * HB + kVColStep];
+#pragma unroll
+    for (int t = 0; t < 2 * HB; ++t) w[t] = 0.f;
+    if (l0 < l1) {
+#pragma unroll
+        for (int t = 0; t < 2 * HB; ++t) {
+            const int L = l0 + t - HB;
+            if (L >= 0 && L < lm) w[t] = col[L];
+        }
+#pragma unroll
+        for (int t = 0; t < HB; ++t) halo[t * kWave] = l1 + t < lm ? col[l1 + t] : 0.f;
+    }
+    __syncthreads();
+    for (int L0 = l0; L0 < l1; L0 += kVColStep) {
+#pragma unroll
+        for (int t = 0; t < kVColStep; ++t) {
+            const int L = L0 + HB + t;
+            w[2 * HB + t] = L < l1 ? col[L] : halo[(L - l1 < HB ? L - l1 : HB - 1) * kWave];
+        }
+        if (L0 >= ilo && L0 + kVColStep <= ihi && L0 + kVColStep <= l1) {
+#pragma unroll
+            for (int q = 0; q < kVColStep; ++q) {
+                float v = 0.f;
+#pragma unroll
+                for (int t = 0; t < NB; ++t) v = __builtin_fmaf(wint.w[t], w[q + t], v);
+                col[L0 + q] = v;
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < kVColStep; ++q) {
+                const int L = L0 + q;
+                if (L >= l1) break;
+                float v = 0.f;
+                const float* c = band + L * NB;
+#pragma unroll
+                for (int t = 0; t < NB; ++t) v = __builtin_fmaf(c[t], w[q + t], v);
+                col[L] = v;
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 2 * HB; ++t) w[t] = w[t + kVColStep];
+    }
+    __syncthreads();
+    if constexpr (VEC) {
+        for (int e = tid; e < n4; e += kBlock) reinterpret_cast<f4*>(dst)[e] = reinterpret_cast<const f4*>(s_col)[e];
+        if (4 * n4 + tid < span) dst[4 * n4 + tid] = s_col[4 * n4 + tid];
+    } else {
+        for (int e = tid; e < span; e += kBlock) dst[e] = s_col[e];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Prolongation P (coarse -> fine), optionally accumulated: the coarse field is
 // read through the half-sample mirror (boco_2d) and interpolated with the
@@ -477,6 +592,20 @@ template <int HB>
 hipError_t launch_vband_h(const VBandArgs& a, hipStream_t st) {
     const bool fixl = a.nfilt == a.K && kBlock % a.lm == 0 && a.K % a.lm == 0;
     const long long N = (long long)a.K * a.npts;
+    // whole columns of a length that spreads them over the LDS banks
+    const long long ncol = a.nfilt == a.K && a.K % a.lm == 0 ? N / a.lm : 0;
+    if constexpr (HB <= kVColMaxHB) if (!fixl && ncol && a.lm % 4 && a.lm <= kVColMaxLm && ncol < (1ll << 31) * kWave) {
+        const dim3 g((unsigned)((ncol + kWave - 1) / kWave));
+        const size_t lds = sizeof(float) * kWave * (a.lm + kVColWaves * HB);
+        // 64 columns start at a multiple of 256 bytes from the base
+        if (((reinterpret_cast<size_t>(a.in) | reinterpret_cast<size_t>(a.out)) & 15) == 0)
+            hipLaunchKernelGGL((vcol_kernel<HB, true>), g, dim3(kBlock), lds, st, a.in, a.out, a.band, a.wint, a.ilo,
+                               a.ihi, a.lm, ncol);
+        else
+            hipLaunchKernelGGL((vcol_kernel<HB, false>), g, dim3(kBlock), lds, st, a.in, a.out, a.band, a.wint, a.ilo,
+                               a.ihi, a.lm, ncol);
+        return hipGetLastError();
+    }
     int cpp = 0, pspan = 0;
     long long nblocks;
     if (a.K > kVSpan) {
