@@ -90,12 +90,14 @@ def build(verbose: bool = False, jobs: int = 0) -> str:
     work = []
     for s in SOURCES:
         work.append((os.path.join(CSRC, s), os.path.join(objdir, s + ".o"), [], verbose))
-    for h in RADIAL_H:
-        work.append((os.path.join(CSRC, RADIAL_TU), os.path.join(objdir, f"radial_h{h}.o"),
-                     [f"-DMGBF_RADIAL_H={h}"], verbose))
-    for h in BALL_H:
+    # the longest compilations first
+    for h in sorted(BALL_H, reverse=True):
         work.append((os.path.join(CSRC, BALL_TU), os.path.join(objdir, f"ball3_h{h}.o"),
                      [f"-DMGBF_BALL_H={h}"], verbose))
+    for h in sorted(RADIAL_H, reverse=True):
+        for part in (1, 2, 0):
+            work.append((os.path.join(CSRC, RADIAL_TU), os.path.join(objdir, f"radial_h{h}_{part}.o"),
+                         [f"-DMGBF_RADIAL_H={h}", f"-DMGBF_RADIAL_PART={part}"], verbose))
     jobs = jobs or min(len(work), max(1, (os.cpu_count() or 4)))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         results = list(ex.map(_compile, work))

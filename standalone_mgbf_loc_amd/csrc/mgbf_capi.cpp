@@ -243,13 +243,49 @@ int drain_timers(mgbf_ctx* c) {
     return status;
 }
 
-// Default rows per wave: the tallest tile that still gives 16384 waves.
+// Default rows per wave of the 3-D and the matrix-core kernels: the tallest
+// tile that still gives 16384 waves.
 int pick_tj(int K, int n, int m, int ti) {
     const long long nkc = (K + 63) / 64;
     const long long ntile_i = (n + ti - 1) / ti;
     int tj = m;
     while (tj > 16 && nkc * ntile_i * ((m + tj - 1) / tj) < 16384) tj = (tj + 1) / 2;
     return tj;
+}
+
+// Default tile of the vector kernel. Two waves a SIMD fit (2048 on the chip)
+// and keep its VALU busy, so a launch takes as long as its rounds of 2048
+// waves, each as long as a wave's rows and the 2H halo rows (of which about
+// three quarters of the work is done): the height with the fewest rounds x
+// rows. 384 x 384 x 320 at H = 6: 112 us at 96 rows (1920 waves), 144 at 128
+// (1440, but no second wave for two fifths of the SIMDs), 138 at 24 (7680);
+// the least height for 16384 waves, the rule before, took 12 rows and 165 us.
+// Generations too small for 2048 waves of 4 rows take 2 columns a lane, half
+// the instructions of a row: 192 x 192 x 32 in 13.2 us against 14.0.
+struct Tile {
+    int ti, tj;
+};
+Tile pick_tile(int kc, int n, int m, int H, bool two, bool even) {
+    constexpr long long kSlots = 2048;
+    auto height = [&](long long segs) {
+        int tj = (int)((m + segs - 1) / segs);
+        if (even && (tj & 1)) tj = tj + 1 <= m ? tj + 1 : tj - 1;
+        return tj < 1 ? 1 : tj;
+    };
+    const long long s4 = mgbf::radial_row_waves(kc, n, 4), s2 = mgbf::radial_row_waves(kc, n, 2);
+    if (two && s4 * ((m + 3) / 4) < kSlots) return {2, height(std::min<long long>(m, std::max(1ll, kSlots / s2)))};
+    Tile best{4, height(1)};
+    double cost = 1e300;
+    for (int segs = 1; segs <= m; ++segs) {
+        const int tj = height(segs);
+        const long long rounds = (s4 * ((m + tj - 1) / tj) + kSlots - 1) / kSlots;
+        const double c = (double)rounds * (tj + 1.5 * H + 2);
+        if (c < cost) {
+            cost = c;
+            best.tj = tj;
+        }
+    }
+    return best;
 }
 
 enum { BAND_VF = 0, BAND_VFT = 1, BAND_VVT = 2 };
@@ -391,13 +427,17 @@ bool fused_ok(const mgbf_ctx* c, int g, int tj, int H) {
     return true;
 }
 
+// Halo rows of the vector pass that carries the restriction: at least the 3
+// its windows need.
+int res_halo(const mgbf_ctx* c) { return std::max(c->s.H, 3); }
+
 // Can the vertical band `which` be fused into the last radial pass of
 // generation 1? Each wave must hold whole columns, and the variant built.
 bool can_fuse_band(const mgbf_ctx* c, int which) {
     const int hb = c->band_hb[which];
     const int lm = c->s.cfg.lm;
     return c->nfilt > 0 && (c->s.exact_disc || c->s.separable) && c->gm > 1 && (64 % lm) == 0 &&
-           (c->K % 64) == 0 &&
+           (c->K % 64) == 0 && c->s.H <= mgbf::kVecMaxBandH &&
            (hb == 3 || hb == 4 || hb == 6 || hb == 8);
 }
 
@@ -557,7 +597,7 @@ int down_sweep(mgbf_ctx* c, const float* u1, float* U, float* T, Weight weight, 
         float* next = last ? nullptr : U + c->goff[g + 1];
         const float* wf = weight == Weight::A ? c->wfield[g] : nullptr;
         const float wc = pass_const(c, g, weight);
-        if (filt && !last && c->fuse >= 3 && !c->aniso[g] && fused_ok(c, g, c->tile_tj[g][3], c->s.H)) {
+        if (filt && !last && c->fuse >= 3 && !c->aniso[g] && fused_ok(c, g, c->tile_tj[g][3], res_halo(c))) {
             CALL(radial(c, g, ug, T + c->goff[g], wf, wc, st, MGBF_T_HFILTT, nullptr, -1, next));
             continue;
         }
@@ -830,9 +870,7 @@ bool plan_ball3(const mgbf::Setup& s, const mgbf_config& cfg, mgbf::Ball3Coef& c
 // procedures 4 and 5: even, so that a restriction can ride in it.
 int rad2d_tj(const mgbf_ctx* c, int g) {
     const int K3 = c->s.dims.km3_all * c->s.cfg.lm;
-    int tj = pick_tj(c->K - K3, c->nx[g], c->ny[g], 4);
-    if (tj & 1) tj = tj + 1 <= c->ny[g] ? tj + 1 : tj - 1;
-    return tj;
+    return pick_tile(c->K - K3, c->nx[g], c->ny[g], c->s.H, false, true).tj;
 }
 
 // The 3-D filter of generation g (F, or F^T with transpose). With `scaled`
@@ -896,9 +934,7 @@ int ball(mgbf_ctx* c, int g, const float* in, float* out, bool transpose, hipStr
         r.klo = K3;
         r.n = c->nx[g];
         r.m = c->ny[g];
-        // the restriction needs 3 halo rows: a narrower filter runs at
-        // half-width 3 with zero taps beyond its own (coef is zero there)
-        r.H = rout ? std::max(c->s.H, 3) : c->s.H;
+        r.H = c->s.H;
         r.TI = 4;
         r.TJ = rad2d_tj(c, g);
         if (rout) {
@@ -968,10 +1004,10 @@ int rad3_down(mgbf_ctx* c, const float* x, float* U, float* T, int g, bool* scal
     float* next = g + 1 < c->gm ? U + c->goff[g + 1] : nullptr;
     const int K3 = c->s.dims.km3_all * c->s.cfg.lm;
     // the streaming pass loads at least 3 halo rows when it restricts
-    // (the 2-D variables after K3 restrict in their radial pass, at H >= 3)
+    // (so does the radial pass of the 2-D variables after K3)
     const bool res = next && c->ball3 && c->fuse >= 3 &&
                      fused_ok(c, g, pick_tj(K3, c->nx[g], c->ny[g], 4), std::max(c->b3H, 3)) &&
-                     (K3 >= c->K || fused_ok(c, g, rad2d_tj(c, g), std::max(c->s.H, 3)));
+                     (K3 >= c->K || fused_ok(c, g, rad2d_tj(c, g), res_halo(c)));
     if (next && !res) CALL(restrict_g(c, g, ug, next, st));
     return ball(c, g, ug, T + c->goff[g], true, st, scaled, nullptr, res ? next : nullptr);
 }
@@ -1298,8 +1334,9 @@ int mgbf_init(const mgbf_config* cfg, int device, mgbf_ctx** out) {
         off += c->gsize[g];
         c->wconst[g] = (float)s.wconst[g];
         for (int kind = 0; kind < 4; ++kind) {
-            c->tile_ti[g][kind] = 4;
-            c->tile_tj[g][kind] = pick_tj(c->K, s.nx[g], s.ny[g], 4);
+            const Tile t = pick_tile(c->K, s.nx[g], s.ny[g], s.H, kind < 2, kind == 3);
+            c->tile_ti[g][kind] = t.ti;
+            c->tile_tj[g][kind] = t.tj;
             if (c->tile_mfma[g][kind]) c->tile_tj[g][kind] = pick_tj(c->K, s.nx[g], s.ny[g], 16);
         }
         // the fused restriction needs an even number of rows per wave
@@ -1835,20 +1872,24 @@ int mgbf_autotune(mgbf_ctx* c, void* stream) {
         for (int kind = 0; kind < 4 && status == MGBF_OK; ++kind) {
             if (kind >= 1 && g + 1 >= c->gm) continue;
             if (kind == 2 && !(g == 0 && c->nfilt > 0 && can_fuse_band(c, vband))) continue;
-            if (kind == 3 && !(c->fuse >= 3 && c->res_ok[g] && c->s.H >= 3)) continue;
+            if (kind == 3 && !(c->fuse >= 3 && c->res_ok[g])) continue;
             const float* coarse = kind == 1 || kind == 2 ? c->ws_u + c->goff[g + 1] : nullptr;
             float* rout = kind == 3 ? c->ws_u + c->goff[g + 1] : nullptr;
             const int band = kind == 2 ? vband : -1;
-            float best = 1e30f;
-            int bti = c->tile_ti[g][kind], btj = c->tile_tj[g][kind], bmf = c->tile_mfma[g][kind];
+            // the fastest tile of the vector kernel and of the matrix cores
+            float best = 1e30f, bestm = 1e30f;
+            int bti = c->tile_ti[g][kind], btj = c->tile_tj[g][kind], btjm = btj;
             const bool try_mfma = mx_ok(c, g, kind);
             // engines: TI = 2, TI = 4 (vector), 16 (matrix cores)
             const int engines[3] = {2, 4, 16};
             for (int en : engines) {
                 if (en == 16 && !try_mfma) continue;
-                if (kind == 3 && en == 2) continue;
+                // 2 columns a lane: the passes without a fused transfer, and
+                // the 4-point prolongation
+                if (en == 2 && (kind >= 2 || (kind == 1 && c->quad))) continue;
                 // waves of one row of tiles (every column tile and k chunk)
-                const long long strip = (long long)((c->K + 63) / 64) * ((n + en - 1) / en) * (en == 16 ? 4 : 1);
+                const long long strip =
+                    en == 16 ? (long long)(c->K / 64) * (n / 16) * 4 : mgbf::radial_row_waves(c->K, n, en);
                 // tile heights: a fixed ladder, and for q = 1 .. 16 the
                 // lowest height whose launch stays within q x 1024 waves
                 // (q / occupancy rounds of the chip's 1024 SIMDs). On a
@@ -1874,9 +1915,9 @@ int mgbf_autotune(mgbf_ctx* c, void* stream) {
                 }
                 for (int q = 0; q < ntj && status == MGBF_OK; ++q) {
                     const int tj = tjs[q];
-                    if (kind == 3 && !fused_ok(c, g, tj, c->s.H)) continue;
+                    if (kind == 3 && !fused_ok(c, g, tj, res_halo(c))) continue;
                     const long long waves = strip * ((m + tj - 1) / tj);
-                    if (waves < 512 && tj != 16) continue;
+                    if (waves < 512 && tj != 16 && tj > 2) continue;
                     c->tile_ti[g][kind] = en == 16 ? 4 : en;
                     c->tile_tj[g][kind] = tj;
                     c->tile_mfma[g][kind] = en == 16 ? 1 : 0;
@@ -1885,17 +1926,29 @@ int mgbf_autotune(mgbf_ctx* c, void* stream) {
                     if (log && status == MGBF_OK)
                         std::fprintf(stderr, "[autotune] gen %d kind %d engine %d TJ %d: %.4f ms\n",
                                      g + 1, kind, en, tj, ms / 3);
-                    if (status == MGBF_OK && ms < best) {
+                    if (status != MGBF_OK) break;
+                    if (en == 16 && ms < bestm) {
+                        bestm = ms;
+                        btjm = tj;
+                    } else if (en != 16 && ms < best) {
                         best = ms;
-                        bti = c->tile_ti[g][kind];
+                        bti = en;
                         btj = tj;
-                        bmf = c->tile_mfma[g][kind];
                     }
                 }
             }
-            c->tile_ti[g][kind] = bti;
-            c->tile_tj[g][kind] = btj;
-            c->tile_mfma[g][kind] = bmf;
+            // a near tie is not left to the noise of three timed passes, which
+            // would choose the engine, and with it the rounding, anew in every
+            // run: a pass over 2^24 values or more goes to the matrix cores
+            // unless they take 1.2x the time, a smaller one (whose 16-column
+            // tiles are the scarcer, the smaller it is) only if they take less
+            // than 0.95x
+            const double tie = (double)c->K * n * m >= 16777216.0 ? 1.2 : 0.95;
+            const bool mx = bestm < 1e30f && bestm <= tie * best;
+            c->tile_ti[g][kind] = mx ? 4 : bti;
+            c->tile_tj[g][kind] = mx ? btjm : btj;
+            if (mx || best < 1e30f) c->tile_mfma[g][kind] = mx ? 1 : 0;
+            best = mx ? bestm : best;
             if (best < 1e30f) kind_ms[kind] = best;
         }
         // the band fused into the last pass (kind 2), or a kind-1 pass and the

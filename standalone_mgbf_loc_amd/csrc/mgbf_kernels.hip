@@ -516,23 +516,32 @@ unsigned grid_for(long long count) {
 
 }  // namespace
 
+// The band runs only over whole columns (lm divides the wave, the wave the
+// stack) after a prolongation, with the half-widths launch_radial_band lists; a
+// weight field or a restriction does not go with a prolongation.
+bool radial_built(const RadialArgs& a) {
+    if (a.mfma || (a.exact_disc && a.separable) || (a.coarse && (a.wfield || a.rout))) return false;
+    if (a.TI != 2 && a.TI != 4) return false;
+    if (!a.band) return true;
+    const bool hb = a.vhb == 3 || a.vhb == 4 || a.vhb == 6 || a.vhb == 8;
+    return hb && (a.exact_disc || a.separable) && a.coarse && !a.klo && a.H <= kVecMaxBandH && a.lm >= 1 && kWave % a.lm == 0 && a.K % kWave == 0;
+}
+
 hipError_t launch_radial(const RadialArgs& a, hipStream_t st) {
     // a k offset takes no band (whole columns are not in the wave) and no
     // matrix-core engine
     if (a.klo < 0 || a.klo >= a.K || (a.klo && (a.mfma || a.band))) return hipErrorInvalidValue;
+#define MGBF_RADIAL_CASE(h)                                   \
+    case h:                                                   \
+        if (a.mfma) return launch_radial_mx_H##h(a, st);      \
+        if (a.exact_disc) return launch_radial_disc_H##h(a, st); \
+        return a.separable ? launch_radial_sep_H##h(a, st) : launch_radial_box_H##h(a, st);
     switch (a.H) {
-        case 1: return launch_radial_H1(a, st);
-        case 2: return launch_radial_H2(a, st);
-        case 3: return launch_radial_H3(a, st);
-        case 4: return launch_radial_H4(a, st);
-        case 5: return launch_radial_H5(a, st);
-        case 6: return launch_radial_H6(a, st);
-        case 7: return launch_radial_H7(a, st);
-        case 8: return launch_radial_H8(a, st);
-        case 9: return launch_radial_H9(a, st);
-        case 10: return launch_radial_H10(a, st);
+        MGBF_RADIAL_CASE(1) MGBF_RADIAL_CASE(2) MGBF_RADIAL_CASE(3) MGBF_RADIAL_CASE(4) MGBF_RADIAL_CASE(5)
+        MGBF_RADIAL_CASE(6) MGBF_RADIAL_CASE(7) MGBF_RADIAL_CASE(8) MGBF_RADIAL_CASE(9) MGBF_RADIAL_CASE(10)
         default: return hipErrorInvalidValue;
     }
+#undef MGBF_RADIAL_CASE
 }
 
 hipError_t launch_ball3(const Ball3Args& a, hipStream_t st) {

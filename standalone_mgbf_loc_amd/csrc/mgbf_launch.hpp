@@ -47,14 +47,14 @@ struct RadialArgs {
     int klo;              // first k filtered (k < klo is left alone): 0, or K3 for
                           // the 2-D variables after the 3-D ones of procedures 4, 5
     int H;                // max(hx, hy)
-    int TI;               // output columns per lane (2 or 4)
+    int TI;               // output columns per lane (2 or 4; 2 runs as 4 where it is not built)
     // matrix-core engine (mgbf_radial_mx.hpp)
     bool mfma;
     const void* bfrag;      // FP16 hi/lo B fragments of the Toeplitz weight bands T_b
     const void* rfrag;      // FP16 B fragments of the x restriction (3 tile classes), or nullptr
     int wexp;               // power-of-two exponent applied to the weights
     int TJ;               // output rows per wavefront
-    // restriction to the next generation fused into the pass (TI = 4, H >= 3)
+    // restriction to the next generation fused into the pass
     float* rout;            // coarse output, or nullptr
     const float4* rytab;    // per fine row: weights into the 6 open coarse rows (2 x float4)
     const int2* rymeta;     // per fine row: lowest open coarse row, rows completed
@@ -75,6 +75,7 @@ struct RadialParams {
     int K, n, m, TJ, lm, nfilt;
     int klo;                  // first k of the pass
     int ntile_i, ntile_j, nitems;
+    int kc, nfw;              // k values laid end to end (0: 64-k chunks), waves per tile row
     // restriction to the next generation fused into the pass (RES)
     float* rout;              // coarse output (n/2 x m/2 x K), or nullptr
     const float4* rytab;      // per fine row: weights into the 6 open coarse rows (2 x float4)
@@ -104,7 +105,28 @@ struct RadialMxParams {
     int ntile_i, ntile_j;
 };
 
-#define MGBF_DECLARE_RADIAL(h) hipError_t launch_radial_H##h(const RadialArgs& a, hipStream_t st);
+// the vector kernel takes the vertical band up to this half-width (beyond it
+// the band's registers do not fit beside the ring and the row buffers)
+constexpr int kVecMaxBandH = 8;
+// Is the vector kernel built for this pass (its taps, epilogues and stack)?
+bool radial_built(const RadialArgs& a);
+// The vector kernel lays the kc stacked values of a tile row's column tiles
+// end to end where chunks of 64 k would idle an eighth of the lanes or more
+// (kc = 32, 65, 130, 2): below that the chunks' order, tiles fastest, reads
+// memory in longer runs (512 x 512 x 520, generation 3: 38 us against 42 us
+// end to end, for 3.4 % idle lanes).
+constexpr bool radial_flattened(int kc) { return kc % 64 && 64ll * ((kc + 63) / 64) * 8 >= 9ll * kc; }
+// Waves of one row of tiles of TI columns.
+constexpr long long radial_row_waves(int kc, int n, int TI) {
+    const long long nt = (n + TI - 1) / TI;
+    return radial_flattened(kc) ? (nt * kc + 63) / 64 : nt * ((kc + 63) / 64);
+}
+
+#define MGBF_DECLARE_RADIAL(h)                                                \
+    hipError_t launch_radial_mx_H##h(const RadialArgs& a, hipStream_t st);    \
+    hipError_t launch_radial_box_H##h(const RadialArgs& a, hipStream_t st);   \
+    hipError_t launch_radial_disc_H##h(const RadialArgs& a, hipStream_t st);  \
+    hipError_t launch_radial_sep_H##h(const RadialArgs& a, hipStream_t st);
 MGBF_DECLARE_RADIAL(1) MGBF_DECLARE_RADIAL(2) MGBF_DECLARE_RADIAL(3) MGBF_DECLARE_RADIAL(4)
 MGBF_DECLARE_RADIAL(5) MGBF_DECLARE_RADIAL(6) MGBF_DECLARE_RADIAL(7) MGBF_DECLARE_RADIAL(8)
 MGBF_DECLARE_RADIAL(9) MGBF_DECLARE_RADIAL(10)

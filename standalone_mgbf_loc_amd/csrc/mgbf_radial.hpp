@@ -1,5 +1,5 @@
-// Radial 2-D beta filter kernel (template), instantiated per half-width H in
-// mgbf_radial_inst.hip.
+// Radial 2-D beta filter kernel (template), instantiated per half-width H and
+// kind of taps in mgbf_radial_inst.hip.
 #pragma once
 
 #include "mgbf_device.hpp"
@@ -14,43 +14,103 @@ __host__ __device__ constexpr int disc_extent(int b) {
     return a;
 }
 
+typedef const __attribute__((address_space(4))) float* ConstF;
+typedef const __attribute__((address_space(4))) int* ConstI;
+
+// A buffer over 2 GiB from `base` (rows are below that size): accesses at
+// kDropped and beyond are out of its range, which the hardware turns into
+// loads of zero and no store.
+constexpr int kDropped = (int)0x80000000;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc_2g(const float* base) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)0x80000000, 0x00020000);
+}
+
+// Row buffers of the input pipeline (one being combined, the others in
+// flight): 4 where the registers of the ring and its epilogues leave room.
+__host__ __device__ constexpr int radial_bufs(int H) { return H <= 6 ? 4 : (H <= 8 ? 3 : 2); }
+
+// One step per ring row S, S+1, .. NR-1 of a turn; the first step past the
+// tile ends it (nested, so that no path rejoins another between two steps and
+// the waits for the row buffers stay exact).
+template <int S, int NR, class F>
+__device__ __forceinline__ void radial_turn(F& step, int rb, int nsteps) {
+    if constexpr (S < NR) {
+        if (rb + S < nsteps) {
+            step(rb + S, std::integral_constant<int, S>{});
+            radial_turn<S + 1, NR>(step, rb, nsteps);
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Radial 2-D beta filter F (gather form, half-sample mirror halo) with the
 // epilogue of its generation:
 //   s(k,i,j) = scale(k,i,j) * sum_{a,b} w(|a|,|b|) in(k, mx(i+a), my(j+b))
 //              [+ (P coarse)(k,i,j)]                       (PRO)
 //   out(k,i,j) = sum_d c(L,d) s(k+d,i,j) over the column    (VHB > 0)
-// scale = wfield (per point) or wconst. One wave computes TI x TJ outputs for
-// its 64 k: input rows stream through registers; for every input row the
-// x-pair sums P_a = v(i+a)+v(i-a) give the per-row partial sums
-// Z_b = sum_a w(a,b) P_a, which are added to the output rows j = r-b and r+b
-// held in a ring of 2H+1 accumulator rows.
+// scale = wfield (per point, not with PRO) or wconst. One wave computes
+// TI x TJ outputs for each of its 64 lanes' k: input rows stream through
+// registers; for every input row the x-pair sums P_a = v(i+a)+v(i-a) give the
+// per-row partial sums Z_b = sum_a w(a,b) P_a, which are added to the output
+// rows j = r-b and r+b held in a ring of accumulator rows.
+// TAPS: the box of w(a,b), the lattice disc a^2 + b^2 < (H+1)^2 with
+// w(a,b) = w(b,a) (one kernel argument each), or the product fx(a) fy(b) (one
+// x-sum per row, fy(b) into rows r+-b).
 // PRO adds the prolongation of the next coarser generation (direct1 on the
 // 2-point mirrored coarse field): a window of 4 x-interpolated coarse rows
 // slides down with the output rows, one new coarse row every other row.
-// VHB applies a vertical band of half-width VHB across the lanes of the wave
-// (each wave then holds whole columns: lm divides 64 and K % 64 == 0).
+// VHB applies a vertical band of half-width VHB across the lanes of the wave.
 // RES restricts the input field to the next generation on the way (R = P^T
 // with the folded edges): every loaded fine row is restricted in x over the
-// wave's 2 coarse columns (interior columns 2I-3 .. 2I+4 with kW8, or
+// tile's 2 coarse columns (interior columns 2I-3 .. 2I+4 with kW8, or
 // 2I-2 .. 2I+3 with the quadratic weights under QP; the 2 columns at each
 // domain edge with the edge table) and added into a shift register of the
 // coarse rows whose windows are open (4 or 3 in the interior, up to 6 next
 // to an edge, with weights from a per-fine-row table there); a coarse row
-// is stored when its window closes.
+// is stored when its window closes. The wave owns coarse rows j0/2 ..
+// (j0+TJ)/2 - 1, whose windows lie inside the rows it loads (checked on the
+// host).
 // QP selects the quadratic transfer (direct2 / adjoint2) for PRO or RES.
-// The wave owns coarse rows j0/2 .. (j0+TJ)/2 - 1, whose windows lie inside
-// the rows it loads (checked on the host).
+//
+// Lanes. Where the stack's Kc = K - klo values fill their last 64-k chunk
+// badly (radial_flattened), the values of all column tiles of a tile row are
+// laid end to end and cut into waves of 64: lane l of wave w works on
+// f = 64 w + l, k = klo + f % Kc of column tile f / Kc. K = 32 fills a wave
+// with two tiles, K = 65 loses nothing where chunks of 64 lose half, and the
+// 2 or 3 two-dimensional variables behind the 3-D ones take 32 or 21 tiles a
+// wave. Column offsets, tile edges and mirrors are per lane (VGPRs) in either
+// layout. The band takes stacks of whole 64-k chunks (with lm dividing 64 a
+// wave then holds whole columns).
+//
+// Input rows are loaded NB - 1 steps ahead into NB register buffers: the VALU
+// is what bounds this kernel (62 operations an output for the H = 6 disc), and
+// with the loads in flight two waves a SIMD keep it 75-90 % busy. The ring has
+// the next multiple of NB above 2H rows, so that ring row and buffer of a step
+// are compile-time constants; the spare rows cost TI registers each.
+// 512 x 512 x 1024 at H = 6: 0.54 ms plain, 0.60 with PRO, 0.70 with PRO and
+// the band of half-width 6, 0.70 with RES (0.60, 0.72, 0.91 and 0.72 when rows
+// were loaded as they were needed, at 3 to 5 waves a SIMD).
+//
+// Partial sums Z_b that reach no output row of the tile are left out: a tile
+// of TJ rows reads TJ + 2H, and of the first and last 2H of them only some b
+// are needed (all of them: 7/3 of the needed work at TJ = 4, H = 6). That
+// makes the short tiles cheap that give a small grid enough waves.
 // ---------------------------------------------------------------------------
-template <int H, int TI, bool DISC, bool PRO, int VHB, bool RES, bool SEP = false, bool QP = false>
+enum { kTapsBox = 0, kTapsDisc = 1, kTapsSep = 2 };
+
+template <int H, int TI, int TAPS, bool PRO, int VHB, bool RES, bool QP>
 __global__ void __launch_bounds__(kBlock) radial_kernel(RadialParams p) {
     static_assert(!QP || PRO || (RES && VHB == 0), "the quadratic transfer rides in PRO or RES");
-    static_assert(!RES || (TI == 4 && H >= 3 && !PRO && VHB == 0), "restriction epilogue shape");
-    static_assert(!(SEP && DISC), "a separable filter is read as a box");
-    constexpr int NR = 2 * H + 1;
-    // columns loaded on each side of the tile: H for the filter, 4 for the
-    // restriction's 8-point stencils at the domain edges
+    static_assert(!RES || (TI == 4 && !PRO && VHB == 0), "restriction epilogue shape");
+    constexpr bool DISC = TAPS == kTapsDisc;
+    constexpr int NB = radial_bufs(H);
+    constexpr int NR = (2 * H + 1 + NB - 1) / NB * NB;
+    // columns and rows loaded on each side: H for the filter, 4 columns and 3
+    // rows for the restriction's 8-point stencils; the D extra rows feed the
+    // restriction only
     constexpr int HL = (RES && H < 4) ? 4 : H;
+    constexpr int HR = (RES && H < 3) ? 3 : H;
+    constexpr int D = HR - H;
     constexpr int NC = TI + 2 * HL;
     constexpr int NCC = TI / 2 + 4;   // coarse columns of the tile (TI even)
     const int lane = threadIdx.x & (kWave - 1);
@@ -58,31 +118,38 @@ __global__ void __launch_bounds__(kBlock) radial_kernel(RadialParams p) {
     const int item = (int)xcd_block(blockIdx.x, gridDim.x) * kWavesPerBlock + wv;
     if (item >= p.nitems) return;
     const int K = p.K, n = p.n, m = p.m;
-    const int ti = item % p.ntile_i;
-    const int rest = item / p.ntile_i;
-    const int tj = rest % p.ntile_j;
-    const int kc = rest / p.ntile_j;
-    const int k = p.klo + kc * kWave + lane;
-    const bool kvalid = k < K;
-    const int kk = kvalid ? k : K - 1;
+    int tj, k, ti;
+    bool valid = true;
+    if (p.kc > 0) {   // the stack end to end over the column tiles
+        const int w = item % p.nfw;
+        tj = item / p.nfw;
+        int f = w * kWave + lane;
+        const int last = p.ntile_i * p.kc - 1;
+        valid = f <= last;
+        f = valid ? f : last;
+        ti = f / p.kc;
+        k = p.klo + f - ti * p.kc;
+    } else {          // 64-k chunks: tiles fastest, chunks slowest
+        ti = item % p.ntile_i;
+        const int rest = item / p.ntile_i;
+        tj = rest % p.ntile_j;
+        k = p.klo + rest / p.ntile_j * kWave + lane;
+        valid = k < K;
+        k = valid ? k : K - 1;
+    }
     const int i0 = ti * TI, j0 = tj * p.TJ;
     const size_t rowstride = (size_t)n * K;
 
-    // byte offsets: per lane k, per column wave-uniform (buffer addressing)
-    const int vk = kk * 4;
-    int soff[NC];
+    // byte offsets inside a row, per lane
+    int voff[NC];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) soff[c] = mirror_half(i0 - HL + c, n) * K * 4;
-    // with the restriction state the column offsets move to VGPRs (per-lane
-    // offsets vk + soff) where that ends the SGPR spills at the same
-    // occupancy (from the compiler's register counts: disc H = 5, 6 and
-    // separable H = 6; elsewhere the VGPRs would cost a wave per SIMD)
-    constexpr bool VOFF = RES && ((DISC && (H == 5 || H == 6)) || (SEP && H == 6));
-    int voff[VOFF ? NC : 1];
-    if constexpr (VOFF) {
+    for (int c = 0; c < NC; ++c) voff[c] = (mirror_half(i0 - HL + c, n) * K + k) * 4;
+    // a lane past the last tile, and columns past the domain, store at an
+    // offset past the buffer's end, which the hardware drops: a branch on a
+    // lane's own condition would cost more than the offsets
+    int vst[TI];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) voff[c] = vk + soff[c];
-    }
+    for (int t = 0; t < TI; ++t) vst[t] = valid && i0 + t < n ? ((i0 + t) * K + k) * 4 : kDropped;
 
     float acc[NR][TI];
 #pragma unroll
@@ -98,28 +165,20 @@ __global__ void __launch_bounds__(kBlock) radial_kernel(RadialParams p) {
     int cbase = 0;
     const int nc = n / 2, mc = m / 2;
     const size_t crow = (size_t)nc * K;
-    auto load_craw = [&](int r, float* dst) {
+    auto load_craw = [&](int r, float* dst) __attribute__((always_inline)) {
         const __amdgpu_buffer_rsrc_t rc = buf_rsrc(p.coarse + (size_t)mirror_half(r, mc) * crow);
 #pragma unroll
-        for (int c = 0; c < NCC; ++c) dst[c] = buf_ld(rc, vk, csoff[c]);
+        for (int c = 0; c < NCC; ++c) dst[c] = buf_ld(rc, csoff[c], 0);
     };
-    // QP: the quadratic transfer (lquart): fine index i reads coarse
-    // (i>>1)-1 .. (i>>1)+1 with Stencil<true>::C[i&1]; the window then starts
-    // at (j>>1)-1 and its fourth row is not read
-    constexpr bool quadp = QP;
-    using SQ = Stencil<true>;
-    auto wbase = [&](int j) { return quadp ? (j >> 1) - 1 : ((j + 1) >> 1) - 2; };
-    auto xinterp = [&](const float* cv, float* dst) {
-        if constexpr (quadp) {
-#pragma unroll
-            for (int t = 0; t < TI; ++t)
-                dst[t] = SQ::C[t & 1][0] * cv[t / 2 + 1] + SQ::C[t & 1][1] * cv[t / 2 + 2] +
-                         SQ::C[t & 1][2] * cv[t / 2 + 3];
-            return;
-        }
+    using PS = Stencil<QP>;
+    auto wbase = [&](int j) { return QP ? (j >> 1) - 1 : ((j + 1) >> 1) - 2; };
+    auto xinterp = [&](const float* cv, float* dst) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < TI; ++t) {
-            if ((t & 1) == 0)
+            if constexpr (QP)
+                dst[t] = PS::C[t & 1][0] * cv[t / 2 + 1] + PS::C[t & 1][1] * cv[t / 2 + 2] +
+                         PS::C[t & 1][2] * cv[t / 2 + 3];
+            else if ((t & 1) == 0)
                 dst[t] = kQc[0] * cv[t / 2] + kQc[1] * cv[t / 2 + 1] + kQc[2] * cv[t / 2 + 2] +
                          kQc[3] * cv[t / 2 + 3];
             else
@@ -128,18 +187,15 @@ __global__ void __launch_bounds__(kBlock) radial_kernel(RadialParams p) {
         }
     };
     if constexpr (PRO) {
-        const int v0 = i0 / 2;
 #pragma unroll
-        for (int c = 0; c < NCC; ++c) csoff[c] = mirror_half(v0 - 2 + c, nc) * K * 4;
+        for (int c = 0; c < NCC; ++c) csoff[c] = (mirror_half(i0 / 2 - 2 + c, nc) * K + k) * 4;
         cbase = wbase(j0);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             load_craw(cbase + u, cvn);
             xinterp(cvn, XV[u]);
         }
-        // prefetch the next coarse row, except where the band epilogue
-        // already presses on the registers
-        if constexpr (VHB == 0) load_craw(cbase + 4, cvn);
+        load_craw(cbase + 4, cvn);
     }
 
     // vertical band coefficients of this lane's level (identity past nfilt)
@@ -154,267 +210,255 @@ __global__ void __launch_bounds__(kBlock) radial_kernel(RadialParams p) {
 #pragma unroll
             for (int d = 0; d < NVB; ++d) vc[d] = d == VHB ? 1.f : 0.f;
         }
+#pragma unroll
+        for (int d = 0; d < NVB; ++d) settle(vc[d]);
     }
 
     const int tj_eff = p.TJ < m - j0 ? p.TJ : m - j0;
-    const int nsteps = tj_eff + 2 * H;
+    const int nsteps = tj_eff + 2 * HR;
 
-    // fused restriction state
-    constexpr int NRC = RES ? TI / 2 : 1;   // coarse columns of the wave
-    constexpr int NQ = 6;                    // open coarse rows at most
+    // fused restriction state; whether the tile lies at the low or the high
+    // edge is per lane
+    constexpr int NRC = RES ? TI / 2 : 1;
+    constexpr int NQ = 6;
     float racc[NQ][NRC];
-    int xcls = 0;                            // 0 interior, 1 left edge, 2 right edge
-    const int Jlo = j0 / 2, Jhi = (j0 + tj_eff) / 2, nc2 = n / 2;
+    const int Jlo = j0 / 2, Jhi = (j0 + tj_eff) / 2;
+    const bool xlow = i0 == 0, xhigh = i0 + TI >= n;
+    int vco[NRC];   // where the coarse columns are stored
     if constexpr (RES) {
+#pragma unroll
+        for (int c = 0; c < NRC; ++c)
+            vco[c] = valid && i0 / 2 + c < nc ? ((i0 / 2 + c) * K + k) * 4 : kDropped;
 #pragma unroll
         for (int q = 0; q < NQ; ++q)
 #pragma unroll
             for (int c = 0; c < NRC; ++c) racc[q][c] = 0.f;
-        xcls = i0 == 0 ? 1 : (i0 + TI >= n ? 2 : 0);
     }
+    auto store_coarse = [&](int J, const float* val) __attribute__((always_inline)) {
+        if (J < Jlo || J >= Jhi) return;
+        const __amdgpu_buffer_rsrc_t ro = buf_rsrc_2g(p.rout + (size_t)J * crow);
+#pragma unroll
+        for (int c = 0; c < NRC; ++c) buf_st(val[c], ro, vco[c], 0);
+    };
 
-    for (int rb = 0; rb < nsteps; rb += NR) {
-        // one step per ring row, unrolled at compile time: the ring index
-        // must be a constant, and a loop the compiler leaves rolled (large
-        // half-widths with the restriction) puts the ring in scratch memory
-        static_for([&](auto S) __attribute__((always_inline)) {
-            constexpr int s = decltype(S)::value;
-            const int rr = rb + s;
-            if (rr < nsteps) {
-                const int r = mirror_half(j0 - H + rr, m);
-                const __amdgpu_buffer_rsrc_t rs = buf_rsrc(p.in + (size_t)r * rowstride);
-                float v[NC];
+    // what step rr needs from memory goes into buffer rr % NB: input row rr
+    // and, with a weight field, the weights of the output row it completes.
+    // Always issued (past the tile's end the last row again), so that the
+    // number of loads behind the ones a step waits for is known.
+    float vb[NB][NC];
+    float wb[RES || !PRO ? NB : 1][TI];
+    auto load_row = [&](int rr, float* v, float* w) __attribute__((always_inline)) {
+        rr = rr < nsteps ? rr : nsteps - 1;
+        const __amdgpu_buffer_rsrc_t rs = buf_rsrc(p.in + (size_t)mirror_half(j0 - HR + rr, m) * rowstride);
 #pragma unroll
-                for (int c = 0; c < NC; ++c) v[c] = VOFF ? buf_ld(rs, voff[c], 0) : buf_ld(rs, vk, soff[c]);
-                if constexpr (RES) {
-                    const int vr = j0 - H + rr;   // fine row, before mirroring
-                    if (vr >= 0 && vr < m) {
-                        using RS = Stencil<QP>;
-                        float xr[NRC];
-                        if (xcls == 0) {          // fine columns 2I+ROFF .. 2I+ROFF+NR-1
+        for (int c = 0; c < NC; ++c) v[c] = buf_ld(rs, voff[c], 0);
+        if constexpr (!PRO) {
+            if (p.wfield) {
+                int jr = rr - D - 2 * H;
+                jr = jr < 0 ? 0 : (jr < tj_eff ? jr : tj_eff - 1);
+                const __amdgpu_buffer_rsrc_t rw = buf_rsrc_2g(p.wfield + (size_t)(j0 + jr) * rowstride);
 #pragma unroll
-                            for (int c = 0; c < NRC; ++c) {
-                                float a = 0.f;
+                for (int t = 0; t < TI; ++t) w[t] = buf_ld(rw, vst[t], 0);   // a dropped column reads zero
+            }
+        }
+    };
 #pragma unroll
-                                for (int t = 0; t < RS::NR; ++t)
-                                    a = __builtin_fmaf(RS::R[t], v[HL + RS::ROFF + 2 * c + t], a);
-                                xr[c] = a;
-                            }
-                        } else if (xcls == 1) {   // fine columns 0 .. 7
+    for (int e = 0; e < NB - 1; ++e) load_row(e, vb[e], wb[PRO ? 0 : e]);
+
+    auto step = [&](const int rr, auto S) __attribute__((always_inline)) {
+        constexpr int s = decltype(S)::value;
+        float* const v = vb[s % NB];
+        load_row(rr + NB - 1, vb[(s + NB - 1) % NB], wb[PRO ? 0 : (s + NB - 1) % NB]);
+        if constexpr (RES) {
+            const int vr = j0 - HR + rr;   // fine row, before mirroring
+            if (vr >= 0 && vr < m) {
+                using RS = Stencil<QP>;
+                float xr[NRC];
 #pragma unroll
-                            for (int c = 0; c < NRC; ++c) {
-                                float a = 0.f;
+                for (int c = 0; c < NRC; ++c) {   // fine columns 2I+ROFF .. 2I+ROFF+NR-1
+                    float a = 0.f;
 #pragma unroll
-                                for (int t = 0; t < 8; ++t)
-                                    a = __builtin_fmaf(QP ? kEdgeRWQ.w[c][t] : kEdgeRW.w[c][t], v[HL + t], a);
-                                xr[c] = a;
-                            }
-                        } else {                  // fine columns n-8 .. n-1
+                    for (int t = 0; t < RS::NR; ++t) a = __builtin_fmaf(RS::R[t], v[HL + RS::ROFF + 2 * c + t], a);
+                    xr[c] = a;
+                }
+                if (__any(xlow || xhigh)) {   // fine columns 0 .. 7, n-8 .. n-1
 #pragma unroll
-                            for (int c = 0; c < NRC; ++c) {
-                                float a = 0.f;
+                    for (int c = 0; c < NRC; ++c) {
+                        float lo = 0.f, hi = 0.f;
 #pragma unroll
-                                for (int t = 0; t < 8; ++t)
-                                    a = __builtin_fmaf(QP ? kEdgeRWQ.w[NRC - 1 - c][7 - t] : kEdgeRW.w[NRC - 1 - c][7 - t],
-                                                       v[HL - 4 + t], a);
-                                xr[c] = a;
-                            }
+                        for (int t = 0; t < 8; ++t) {
+                            lo = __builtin_fmaf(QP ? kEdgeRWQ.w[c][t] : kEdgeRW.w[c][t], v[HL + t], lo);
+                            hi = __builtin_fmaf(QP ? kEdgeRWQ.w[NRC - 1 - c][7 - t] : kEdgeRW.w[NRC - 1 - c][7 - t],
+                                                v[HL - 4 + t], hi);
                         }
-                        if (vr >= 8 && vr <= m - 9) {
-                            // interior fine row: coarse rows jb .. jb+NO-1 are
-                            // open (windows 2J+ROFF .. 2J+ROFF+NR-1). A row of
-                            // parity CP is the last of row jb's window: it reads
-                            // taps NR-1, NR-3, .. of the open windows and closes
-                            // row jb; a row of the other parity reads taps
-                            // NR-2, NR-4, .. (4-point: even rows close, quadratic:
-                            // odd rows)
-                            constexpr int NO = RS::NR / 2;
-                            constexpr int CP = (RS::ROFF + RS::NR - 1) & 1;
-                            const bool closes = (vr & 1) == CP;
-                            float yw[NO];
-#pragma unroll
-                            for (int q = 0; q < NO; ++q)
-                                yw[q] = closes ? RS::R[RS::NR - 1 - 2 * q] : RS::R[RS::NR - 2 - 2 * q];
-#pragma unroll
-                            for (int q = 0; q < NO; ++q)
-#pragma unroll
-                                for (int c = 0; c < NRC; ++c)
-                                    racc[q][c] = __builtin_fmaf(yw[q], xr[c], racc[q][c]);
-                            if (closes) {
-                                const int J = (vr - RS::ROFF - RS::NR + 1) >> 1;
-                                if (J >= Jlo && J < Jhi && kvalid) {
-                                    const __amdgpu_buffer_rsrc_t ro =
-                                        buf_rsrc(p.rout + (size_t)K * ((size_t)(i0 / 2) + (size_t)nc2 * J));
-#pragma unroll
-                                    for (int c = 0; c < NRC; ++c) {
-                                        if (i0 / 2 + c < nc2) buf_st(racc[0][c], ro, vk, c * K * 4);
-                                    }
-                                }
-                                // slots NO .. 5 stay empty between the edges
-#pragma unroll
-                                for (int q = 0; q + 1 < NO; ++q)
-#pragma unroll
-                                    for (int c = 0; c < NRC; ++c) racc[q][c] = racc[q + 1][c];
-#pragma unroll
-                                for (int c = 0; c < NRC; ++c) racc[NO - 1][c] = 0.f;
-                            }
-                        } else {
-                            // rows next to an edge: weights and closing rows
-                            // from the table
-                            const float4 ya = p.rytab[2 * vr], yb = p.rytab[2 * vr + 1];
-                            const float yw[NQ] = {ya.x, ya.y, ya.z, ya.w, yb.x, yb.y};
-                            const int2 meta = p.rymeta[vr];
-#pragma unroll
-                            for (int q = 0; q < NQ; ++q)
-#pragma unroll
-                                for (int c = 0; c < NRC; ++c)
-                                    racc[q][c] = __builtin_fmaf(yw[q], xr[c], racc[q][c]);
-                            // coarse rows meta.x .. meta.x + meta.y - 1 close here
-#pragma unroll
-                            for (int e = 0; e < NQ; ++e) {
-                                const int J = meta.x + e;
-                                if (e < meta.y && J >= Jlo && J < Jhi && kvalid) {
-                                    const __amdgpu_buffer_rsrc_t ro =
-                                        buf_rsrc(p.rout + (size_t)K * ((size_t)(i0 / 2) + (size_t)nc2 * J));
-#pragma unroll
-                                    for (int c = 0; c < NRC; ++c) {
-                                        if (i0 / 2 + c < nc2) buf_st(racc[e][c], ro, vk, c * K * 4);
-                                    }
-                                }
-                            }
-#pragma unroll
-                            for (int sft = 1; sft <= NQ; ++sft) {
-                                if (meta.y == sft) {
-#pragma unroll
-                                    for (int q = 0; q < NQ; ++q)
-#pragma unroll
-                                        for (int c = 0; c < NRC; ++c)
-                                            racc[q][c] = q + sft < NQ ? racc[q + sft < NQ ? q + sft : 0][c] : 0.f;
-                                }
-                            }
-                        }
+                        xr[c] = xlow ? lo : (xhigh ? hi : xr[c]);
                     }
                 }
+                // the row enters the open coarse rows: inside, NO of them,
+                // with the stencil's odd or even taps, and a row of parity CP
+                // closes the oldest; in the 8 rows next to an edge up to 6,
+                // with weights and closing rows from the table (constant
+                // address space: scalar loads, which leave the count of row
+                // loads in flight alone)
+                constexpr int NO = RS::NR / 2;
+                constexpr int CP = (RS::ROFF + RS::NR - 1) & 1;
+                const bool edge = vr < 8 || vr > m - 9;
+                float yw[NQ];
+                int J, nclose;
+                if (edge) {
+                    const ConstF ry = (ConstF)(size_t)p.rytab + 8 * vr;
+                    const ConstI rm = (ConstI)(size_t)p.rymeta + 2 * vr;
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) yw[q] = ry[q];
+                    J = rm[0];
+                    nclose = rm[1];
+                } else {
+                    const bool closes = (vr & 1) == CP;
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q)
+                        yw[q] = q >= NO ? 0.f : (closes ? RS::R[RS::NR - 1 - 2 * (q % NO)] : RS::R[RS::NR - 2 - 2 * (q % NO)]);
+                    J = (vr - RS::ROFF - RS::NR + 1) >> 1;
+                    nclose = closes ? 1 : 0;
+                }
+#pragma unroll
+                for (int q = 0; q < NO; ++q)
+#pragma unroll
+                    for (int c = 0; c < NRC; ++c) racc[q][c] = __builtin_fmaf(yw[q], xr[c], racc[q][c]);
+                if (edge) {
+#pragma unroll
+                    for (int q = NO; q < NQ; ++q)
+#pragma unroll
+                        for (int c = 0; c < NRC; ++c) racc[q][c] = __builtin_fmaf(yw[q], xr[c], racc[q][c]);
+                }
+#pragma unroll 1
+                for (; nclose > 0; --nclose, ++J) {
+                    store_coarse(J, racc[0]);
+#pragma unroll
+                    for (int q = 0; q + 1 < NQ; ++q)
+#pragma unroll
+                        for (int c = 0; c < NRC; ++c) racc[q][c] = racc[q + 1][c];
+#pragma unroll
+                    for (int c = 0; c < NRC; ++c) racc[NQ - 1][c] = 0.f;
+                }
+            }
+        }
+        // filter row f, the centre of output row c = f - H: Z_b reaches output
+        // rows c - b and c + b, one of which must lie in the tile
+        const int f = rr - D;
+        if (D > 0 && (f < 0 || f >= tj_eff + 2 * H)) return;
+        const int ctr = f - H;
+        const int blo = ctr < 0 ? -ctr : (ctr >= tj_eff ? ctr - tj_eff + 1 : 0);
+        const int up = tj_eff - 1 - ctr;
+        int bhi = ctr < 0 ? up : (ctr >= tj_eff ? ctr : (ctr > up ? ctr : up));
+        bhi = bhi < H ? bhi : H;
+        const unsigned need = (2u << bhi) - (1u << blo);   // bit b: Z_b is needed
+        constexpr int sf = s + 2 * NR - D;   // ring row of f, modulo NR
+        if constexpr (TAPS == kTapsSep) {
+            // w(a,b) = fx(a) fy(b): one x-sum per row, fy(b) into rows f+-b
+            float q[TI];
+#pragma unroll
+            for (int t = 0; t < TI; ++t) {
+                q[t] = p.W.w[0][0] * v[t + HL];
+#pragma unroll
+                for (int a = 1; a <= H; ++a)
+                    q[t] = __builtin_fmaf(p.W.w[0][a], v[t + HL + a] + v[t + HL - a], q[t]);
+            }
+#pragma unroll
+            for (int b = 0; b <= H; ++b) {
+                if (!(need >> b & 1)) continue;
 #pragma unroll
                 for (int t = 0; t < TI; ++t) {
-                    float P[H + 1];
-                    P[0] = v[t + HL];
-#pragma unroll
-                    for (int a = 1; a <= H; ++a) P[a] = v[t + HL + a] + v[t + HL - a];
-                    if constexpr (SEP) {
-                        // w(a,b) = fx(a) fy(b): one x-sum per row, fy(b) into rows r+-b
-                        float q = p.W.w[0][0] * P[0];
-#pragma unroll
-                        for (int a = 1; a <= H; ++a) q = __builtin_fmaf(p.W.w[0][a], P[a], q);
-#pragma unroll
-                        for (int b = 0; b <= H; ++b) {
-                            acc[(s + b) % NR][t] = __builtin_fmaf(p.W.w[1][b], q, acc[(s + b) % NR][t]);
-                            if (b > 0)
-                                acc[(s + NR - b) % NR][t] =
-                                    __builtin_fmaf(p.W.w[1][b], q, acc[(s + NR - b) % NR][t]);
-                        }
-                        continue;
-                    }
-#pragma unroll
-                    for (int b = 0; b <= H; ++b) {
-                        const int A = DISC ? disc_extent<H>(b) : H;
-                        // on the disc w(a,b) = w(b,a): one kernel argument each
-                        float z = p.W.w[DISC ? 0 : b][DISC ? b : 0] * P[0];
-#pragma unroll
-                        for (int a = 1; a <= H; ++a)
-                            if (a <= A)
-                                z = __builtin_fmaf(p.W.w[DISC && a < b ? a : b][DISC && a < b ? b : a],
-                                                   P[a], z);
-                        acc[(s + b) % NR][t] += z;
-                        if (b > 0) acc[(s + NR - b) % NR][t] += z;
-                    }
+                    acc[(sf + b) % NR][t] = __builtin_fmaf(p.W.w[1][b], q[t], acc[(sf + b) % NR][t]);
+                    if (b > 0) acc[(sf - b) % NR][t] = __builtin_fmaf(p.W.w[1][b], q[t], acc[(sf - b) % NR][t]);
                 }
-                // output row j = j0 + rr - 2H is complete
-                const int jrel = rr - 2 * H;
-                constexpr int slot_off = NR - H;   // (s - H) mod NR
-                if (jrel >= 0 && jrel < tj_eff) {
-                    const int j = j0 + jrel;
-                    const size_t rowoff = (size_t)j * rowstride + (size_t)i0 * K;
-                    float o[TI];
-                    if (p.wfield) {
-                        const __amdgpu_buffer_rsrc_t rw = buf_rsrc(p.wfield + rowoff);
-#pragma unroll
-                        for (int t = 0; t < TI; ++t) {
-                            const int tc = i0 + t < n ? t : n - 1 - i0;
-                            o[t] = buf_ld(rw, vk, tc * K * 4) * acc[(s + slot_off) % NR][t];
-                        }
-                    } else {
-#pragma unroll
-                        for (int t = 0; t < TI; ++t) o[t] = p.wconst * acc[(s + slot_off) % NR][t];
-                    }
-                    if constexpr (PRO) {
-                        const int nb = wbase(j);
-                        if (nb != cbase) {   // the window moves down one coarse row
-#pragma unroll
-                            for (int u = 0; u < 3; ++u)
-#pragma unroll
-                                for (int t = 0; t < TI; ++t) XV[u][t] = XV[u + 1][t];
-                            if constexpr (VHB == 0) {
-                                xinterp(cvn, XV[3]);
-                                load_craw(nb + 4, cvn);
-                            } else {
-                                load_craw(nb + 3, cvn);
-                                xinterp(cvn, XV[3]);
-                            }
-                            cbase = nb;
-                        }
-                        const bool oj = (j & 1) != 0;
-                        float y0, y1, y2, y3;
-                        if constexpr (quadp) {
-                            y0 = oj ? SQ::C[1][0] : SQ::C[0][0];
-                            y1 = oj ? SQ::C[1][1] : SQ::C[0][1];
-                            y2 = oj ? SQ::C[1][2] : SQ::C[0][2];
-                            y3 = 0.f;
-                        } else {
-                            y0 = oj ? kPc[0] : kQc[0];
-                            y1 = oj ? kPc[1] : kQc[1];
-                            y2 = oj ? kPc[2] : kQc[2];
-                            y3 = oj ? kPc[3] : kQc[3];
-                        }
-#pragma unroll
-                        for (int t = 0; t < TI; ++t)
-                            o[t] += y0 * XV[0][t] + y1 * XV[1][t] + y2 * XV[2][t] + y3 * XV[3][t];
-                    }
-                    if constexpr (VHB > 0) {
-                        // the band over the lanes: level k+d sits in lane
-                        // lane+d, reached by d single-lane wave shifts (DPP);
-                        // lanes shifted in from outside the wave read 0 and
-                        // meet a zero band coefficient, as do lanes of the
-                        // neighbouring column
-#pragma unroll
-                        for (int t = 0; t < TI; ++t) {
-                            float up = o[t], dn = o[t];
-                            float rsum = vc[VHB] * o[t];
-#pragma unroll
-                            for (int d = 1; d <= VHB; ++d) {
-                                up = lane_from_above(up);
-                                dn = lane_from_below(dn);
-                                rsum = __builtin_fmaf(vc[VHB + d], up, rsum);
-                                rsum = __builtin_fmaf(vc[VHB - d], dn, rsum);
-                            }
-                            o[t] = rsum;
-                        }
-                    }
-                    if (kvalid) {
-                        const __amdgpu_buffer_rsrc_t ro = buf_rsrc(p.out + rowoff);
-#pragma unroll
-                        for (int t = 0; t < TI; ++t)
-                            if (i0 + t < n) buf_st(o[t], ro, vk, t * K * 4);
-                    }
-                }
-#pragma unroll
-                for (int t = 0; t < TI; ++t) acc[(s + slot_off) % NR][t] = 0.f;
             }
-        }, std::make_integer_sequence<int, NR>{});
-    }
+        } else {
+            float P[TI][H + 1];
+#pragma unroll
+            for (int t = 0; t < TI; ++t) {
+                P[t][0] = v[t + HL];
+#pragma unroll
+                for (int a = 1; a <= H; ++a) P[t][a] = v[t + HL + a] + v[t + HL - a];
+            }
+#pragma unroll
+            for (int b = 0; b <= H; ++b) {
+                if (!(need >> b & 1)) continue;
+                const int A = DISC ? disc_extent<H>(b) : H;
+#pragma unroll
+                for (int t = 0; t < TI; ++t) {
+                    // on the disc w(a,b) = w(b,a): one kernel argument each
+                    float z = p.W.w[DISC ? 0 : b][DISC ? b : 0] * P[t][0];
+#pragma unroll
+                    for (int a = 1; a <= H; ++a)
+                        if (a <= A)
+                            z = __builtin_fmaf(p.W.w[DISC && a < b ? a : b][DISC && a < b ? b : a], P[t][a], z);
+                    acc[(sf + b) % NR][t] += z;
+                    if (b > 0) acc[(sf - b) % NR][t] += z;
+                }
+            }
+        }
+        // output row j = j0 + f - 2H is complete
+        const int jrel = f - 2 * H;
+        constexpr int os = (sf - H) % NR;
+        if (jrel >= 0 && jrel < tj_eff) {
+            const int j = j0 + jrel;
+            float o[TI];
+#pragma unroll
+            for (int t = 0; t < TI; ++t) o[t] = (!PRO && p.wfield ? wb[PRO ? 0 : s % NB][t] : p.wconst) * acc[os][t];
+            if constexpr (PRO) {
+                const int nb = wbase(j);
+                if (nb != cbase) {   // the window moves down one coarse row
+#pragma unroll
+                    for (int u = 0; u < 3; ++u)
+#pragma unroll
+                        for (int t = 0; t < TI; ++t) XV[u][t] = XV[u + 1][t];
+                    xinterp(cvn, XV[3]);
+                    load_craw(nb + 4, cvn);
+                    cbase = nb;
+                }
+                const bool oj = (j & 1) != 0;
+                constexpr int NP = PS::NP;
+                float y[NP];
+#pragma unroll
+                for (int u = 0; u < NP; ++u) y[u] = oj ? PS::C[1][u] : PS::C[0][u];
+#pragma unroll
+                for (int t = 0; t < TI; ++t) {
+                    if constexpr (QP)
+                        o[t] += y[0] * XV[0][t] + y[1] * XV[1][t] + y[2] * XV[2][t];
+                    else
+                        o[t] += y[0] * XV[0][t] + y[1] * XV[1][t] + y[2] * XV[2][t] + y[NP - 1] * XV[3][t];
+                }
+            }
+            if constexpr (VHB > 0) {
+                // the band over the lanes: level k+d sits in lane lane+d,
+                // reached by d single-lane wave shifts (DPP); lanes shifted in
+                // from outside the wave read 0 and meet a zero band
+                // coefficient, as do lanes of the neighbouring column
+#pragma unroll
+                for (int t = 0; t < TI; ++t) {
+                    float lu = o[t], ld = o[t];
+                    float rsum = vc[VHB] * o[t];
+#pragma unroll
+                    for (int d = 1; d <= VHB; ++d) {
+                        lu = lane_from_above(lu);
+                        ld = lane_from_below(ld);
+                        rsum = __builtin_fmaf(vc[VHB + d], lu, rsum);
+                        rsum = __builtin_fmaf(vc[VHB - d], ld, rsum);
+                    }
+                    o[t] = rsum;
+                }
+            }
+            const __amdgpu_buffer_rsrc_t ro = buf_rsrc_2g(p.out + (size_t)j * rowstride);
+#pragma unroll
+            for (int t = 0; t < TI; ++t) buf_st(o[t], ro, vst[t], 0);
+        }
+#pragma unroll
+        for (int t = 0; t < TI; ++t) acc[os][t] = 0.f;
+    };
+    for (int rb = 0; rb < nsteps; rb += NR) radial_turn<0, NR>(step, rb, nsteps);
 }
 
-template <int H, int TI, bool DISC, bool PRO, int VHB, bool RES = false, bool SEP = false, bool QP = false>
+template <int H, int TI, int TAPS, bool PRO, int VHB, bool RES, bool QP>
 hipError_t launch_radial_variant(const RadialArgs& a, hipStream_t st) {
     RadialParams p{};
     p.in = a.in;
@@ -436,95 +480,51 @@ hipError_t launch_radial_variant(const RadialArgs& a, hipStream_t st) {
     p.rymeta = a.rymeta;
     p.ntile_i = (a.n + TI - 1) / TI;
     p.ntile_j = (a.m + a.TJ - 1) / a.TJ;
-    const int nkc = (a.K - a.klo + kWave - 1) / kWave;
-    const long long nitems = (long long)p.ntile_i * p.ntile_j * nkc;
+    const int kc = a.K - a.klo;
+    p.kc = radial_flattened(kc) ? kc : 0;
+    const long long row = radial_row_waves(kc, a.n, TI);
+    p.nfw = (int)row;
+    const long long nitems = row * p.ntile_j;
+    if (nitems >= (1ll << 31) || (long long)p.ntile_i * kc >= (1ll << 31)) return hipErrorInvalidValue;
     p.nitems = (int)nitems;
     const unsigned nblocks = (unsigned)((nitems + kWavesPerBlock - 1) / kWavesPerBlock);
-    hipLaunchKernelGGL((radial_kernel<H, TI, DISC, PRO, VHB, RES, SEP, QP>), dim3(nblocks), dim3(kBlock), 0, st,
-                       p);
+    hipLaunchKernelGGL((radial_kernel<H, TI, TAPS, PRO, VHB, RES, QP>), dim3(nblocks), dim3(kBlock), 0, st, p);
     return hipGetLastError();
 }
 
-// Dispatch over the built variants for one H and tile width TI.
-template <int H, int TI>
-hipError_t launch_radial_ti(const RadialArgs& a, hipStream_t st) {
-    const bool pro = a.coarse != nullptr;
-    const int vhb = a.band ? a.vhb : 0;
-    if (a.quad && pro) {   // the quadratic prolongation epilogue, with or without band
-        if (a.separable) {
-            switch (vhb) {
-                case 0: return launch_radial_variant<H, TI, false, true, 0, false, true, true>(a, st);
-                case 3: return launch_radial_variant<H, TI, false, true, 3, false, true, true>(a, st);
-                case 4: return launch_radial_variant<H, TI, false, true, 4, false, true, true>(a, st);
-                case 6: return launch_radial_variant<H, TI, false, true, 6, false, true, true>(a, st);
-                case 8: return launch_radial_variant<H, TI, false, true, 8, false, true, true>(a, st);
-                default: return hipErrorInvalidValue;
-            }
-        }
-        if (!a.exact_disc) {
-            if (vhb) return hipErrorInvalidValue;
-            return launch_radial_variant<H, TI, false, true, 0, false, false, true>(a, st);
-        }
-        switch (vhb) {
-            case 0: return launch_radial_variant<H, TI, true, true, 0, false, false, true>(a, st);
-            case 3: return launch_radial_variant<H, TI, true, true, 3, false, false, true>(a, st);
-            case 4: return launch_radial_variant<H, TI, true, true, 4, false, false, true>(a, st);
-            case 6: return launch_radial_variant<H, TI, true, true, 6, false, false, true>(a, st);
-            case 8: return launch_radial_variant<H, TI, true, true, 8, false, false, true>(a, st);
-            default: return hipErrorInvalidValue;
-        }
-    }
-    if (a.rout) {   // restriction epilogue: plain pass, 4 columns per lane, H >= 3
-        if constexpr (TI == 4 && H >= 3) {
-            if (pro || vhb) return hipErrorInvalidValue;
-            if (a.quad) {
-                if (a.separable) return launch_radial_variant<H, 4, false, false, 0, true, true, true>(a, st);
-                return a.exact_disc ? launch_radial_variant<H, 4, true, false, 0, true, false, true>(a, st)
-                                    : launch_radial_variant<H, 4, false, false, 0, true, false, true>(a, st);
-            }
-            if (a.separable) return launch_radial_variant<H, 4, false, false, 0, true, true>(a, st);
-            return a.exact_disc ? launch_radial_variant<H, 4, true, false, 0, true>(a, st)
-                                : launch_radial_variant<H, 4, false, false, 0, true>(a, st);
-        } else {
-            return hipErrorInvalidValue;
-        }
-    }
-    if (a.separable) {
-        if (vhb == 0) return pro ? launch_radial_variant<H, TI, false, true, 0, false, true>(a, st)
-                                 : launch_radial_variant<H, TI, false, false, 0, false, true>(a, st);
-        if (!pro) return hipErrorInvalidValue;
-        switch (vhb) {
-            case 3: return launch_radial_variant<H, TI, false, true, 3, false, true>(a, st);
-            case 4: return launch_radial_variant<H, TI, false, true, 4, false, true>(a, st);
-            case 6: return launch_radial_variant<H, TI, false, true, 6, false, true>(a, st);
-            case 8: return launch_radial_variant<H, TI, false, true, 8, false, true>(a, st);
-            default: return hipErrorInvalidValue;
-        }
-    }
-    if (a.exact_disc) {
-        if (vhb == 0) return pro ? launch_radial_variant<H, TI, true, true, 0>(a, st)
-                                 : launch_radial_variant<H, TI, true, false, 0>(a, st);
-        if (!pro) return hipErrorInvalidValue;
-        switch (vhb) {
-            case 3: return launch_radial_variant<H, TI, true, true, 3>(a, st);
-            case 4: return launch_radial_variant<H, TI, true, true, 4>(a, st);
-            case 6: return launch_radial_variant<H, TI, true, true, 6>(a, st);
-            case 8: return launch_radial_variant<H, TI, true, true, 8>(a, st);
-            default: return hipErrorInvalidValue;
-        }
-    }
-    if (vhb != 0) return hipErrorInvalidValue;
-    return pro ? launch_radial_variant<H, TI, false, true, 0>(a, st)
-               : launch_radial_variant<H, TI, false, false, 0>(a, st);
+// The pass kinds; radial_built, checked here, lists what is built.
+template <int H, int TAPS, int VHB>
+hipError_t launch_radial_band(const RadialArgs& a, hipStream_t st) {
+    if constexpr (H <= kVecMaxBandH && TAPS != kTapsBox)
+        return a.quad ? launch_radial_variant<H, 4, TAPS, true, VHB, false, true>(a, st)
+                      : launch_radial_variant<H, 4, TAPS, true, VHB, false, false>(a, st);
+    else
+        return hipErrorInvalidValue;
 }
 
-template <int H>
-hipError_t launch_radial_h(const RadialArgs& a, hipStream_t st) {
-    switch (a.TI) {
-        case 2: return launch_radial_ti<H, 2>(a, st);
-        case 4: return launch_radial_ti<H, 4>(a, st);
-        default: return hipErrorInvalidValue;
+template <int H, int TAPS>
+hipError_t launch_radial_taps(const RadialArgs& a, hipStream_t st) {
+    if (!radial_built(a) || a.TJ < 1 || (TAPS == kTapsDisc) != a.exact_disc || (TAPS == kTapsSep) != a.separable)
+        return hipErrorInvalidValue;
+    if (a.band) {
+        switch (a.vhb) {
+            case 3: return launch_radial_band<H, TAPS, 3>(a, st);
+            case 4: return launch_radial_band<H, TAPS, 4>(a, st);
+            case 6: return launch_radial_band<H, TAPS, 6>(a, st);
+            case 8: return launch_radial_band<H, TAPS, 8>(a, st);
+            default: return hipErrorInvalidValue;
+        }
     }
+    if (a.rout)
+        return a.quad ? launch_radial_variant<H, 4, TAPS, false, 0, true, true>(a, st)
+                      : launch_radial_variant<H, 4, TAPS, false, 0, true, false>(a, st);
+    if constexpr (TAPS != kTapsBox) {   // 2 columns a lane, for the smallest launches
+        if (a.TI == 2 && !a.coarse) return launch_radial_variant<H, 2, TAPS, false, 0, false, false>(a, st);
+        if (a.TI == 2 && !a.quad) return launch_radial_variant<H, 2, TAPS, true, 0, false, false>(a, st);
+    }
+    if (!a.coarse) return launch_radial_variant<H, 4, TAPS, false, 0, false, false>(a, st);
+    return a.quad ? launch_radial_variant<H, 4, TAPS, true, 0, false, true>(a, st)
+                  : launch_radial_variant<H, 4, TAPS, true, 0, false, false>(a, st);
 }
 
 }  // namespace mgbf
