@@ -265,20 +265,19 @@ int pick_tj(int K, int n, int m, int ti) {
 struct Tile {
     int ti, tj;
 };
-Tile pick_tile(int kc, int n, int m, int H, bool two, bool even) {
-    constexpr long long kSlots = 2048;
+Tile pick_tile(int kc, int n, int m, int H, bool two, bool even, long long slots = 2048) {
     auto height = [&](long long segs) {
         int tj = (int)((m + segs - 1) / segs);
         if (even && (tj & 1)) tj = tj + 1 <= m ? tj + 1 : tj - 1;
         return tj < 1 ? 1 : tj;
     };
     const long long s4 = mgbf::radial_row_waves(kc, n, 4), s2 = mgbf::radial_row_waves(kc, n, 2);
-    if (two && s4 * ((m + 3) / 4) < kSlots) return {2, height(std::min<long long>(m, std::max(1ll, kSlots / s2)))};
+    if (two && s4 * ((m + 3) / 4) < slots) return {2, height(std::min<long long>(m, std::max(1ll, slots / s2)))};
     Tile best{4, height(1)};
     double cost = 1e300;
     for (int segs = 1; segs <= m; ++segs) {
         const int tj = height(segs);
-        const long long rounds = (s4 * ((m + tj - 1) / tj) + kSlots - 1) / kSlots;
+        const long long rounds = (s4 * ((m + tj - 1) / tj) + slots - 1) / slots;
         const double c = (double)rounds * (tj + 1.5 * H + 2);
         if (c < cost) {
             cost = c;
@@ -867,10 +866,14 @@ bool plan_ball3(const mgbf::Setup& s, const mgbf_config& cfg, mgbf::Ball3Coef& c
 }
 
 // Rows per wave of the radial pass over the 2-D variables (k >= K3) of
-// procedures 4 and 5: even, so that a restriction can ride in it.
+// procedures 4 and 5: even, so that a restriction can ride in it. A few values
+// a column, a stack apart, are a cache line a lane: the lines a CU can ask for
+// bound the pass, not its VALU, and more than two waves a CU only repeat halo
+// rows (768 x 768 x 2 of 258: 57 us at 12 rows, 384 waves; 64 at 8 and at 16;
+// 91 at 4).
 int rad2d_tj(const mgbf_ctx* c, int g) {
     const int K3 = c->s.dims.km3_all * c->s.cfg.lm;
-    return pick_tile(c->K - K3, c->nx[g], c->ny[g], c->s.H, false, true).tj;
+    return std::max(pick_tile(c->K - K3, c->nx[g], c->ny[g], c->s.H, false, true, 512).tj, std::min(c->ny[g], 4));
 }
 
 // The 3-D filter of generation g (F, or F^T with transpose). With `scaled`

@@ -76,6 +76,7 @@ struct RadialParams {
     int klo;                  // first k of the pass
     int ntile_i, ntile_j, nitems;
     int kc, nfw;              // k values laid end to end (0: 64-k chunks), waves per tile row
+    int wpb;                  // waves per block
     // restriction to the next generation fused into the pass (RES)
     float* rout;              // coarse output (n/2 x m/2 x K), or nullptr
     const float4* rytab;      // per fine row: weights into the 6 open coarse rows (2 x float4)
