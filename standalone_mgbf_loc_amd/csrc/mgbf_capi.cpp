@@ -243,8 +243,8 @@ int drain_timers(mgbf_ctx* c) {
     return status;
 }
 
-// Default rows per wave of the 3-D and the matrix-core kernels: the tallest
-// tile that still gives 16384 waves.
+// Default rows per wave of the matrix-core kernel: the tallest tile that still
+// gives 16384 waves.
 int pick_tj(int K, int n, int m, int ti) {
     const long long nkc = (K + 63) / 64;
     const long long ntile_i = (n + ti - 1) / ti;
@@ -265,7 +265,8 @@ int pick_tj(int K, int n, int m, int ti) {
 struct Tile {
     int ti, tj;
 };
-Tile pick_tile(int kc, int n, int m, int H, bool two, bool even, long long slots = 2048) {
+Tile pick_tile(int kc, int n, int m, int H, bool two, bool even, long long slots = 2048,
+               int cap = 1 << 30) {
     auto height = [&](long long segs) {
         int tj = (int)((m + segs - 1) / segs);
         if (even && (tj & 1)) tj = tj + 1 <= m ? tj + 1 : tj - 1;
@@ -277,6 +278,7 @@ Tile pick_tile(int kc, int n, int m, int H, bool two, bool even, long long slots
     double cost = 1e300;
     for (int segs = 1; segs <= m; ++segs) {
         const int tj = height(segs);
+        if (tj > cap) continue;
         const long long rounds = (s4 * ((m + tj - 1) / tj) + slots - 1) / slots;
         const double c = (double)rounds * (tj + 1.5 * H + 2);
         if (c < cost) {
@@ -865,6 +867,19 @@ bool plan_ball3(const mgbf::Setup& s, const mgbf_config& cfg, mgbf::Ball3Coef& c
     return lm >= 2 * HZ + 2;
 }
 
+// Rows per wave of the 3-D kernel: as pick_tile's, in rounds of the 3 waves a
+// SIMD that fit there, up to 96 rows. 768 x 768 x 256 at half-width 3, with the
+// restriction and with the prolongation: 485 and 456 us at 96 rows, 540 and 498
+// at 24, the least height for 16384 waves, the rule before; 384 x 384: 142 and
+// 129 at 48 (one round), 161 and 146 at 16. On 1536 x 1536 x 512 the waves of
+// 192 rows and more drift too far apart to share rows in the L2: an application
+// takes 9.03 ms at 96, 9.41 at 192, 9.98 at 24 (7.00, 7.39, 7.06 for the line
+// procedure).
+int ball3_tj(const mgbf_ctx* c, int g) {
+    const int chunks = (c->s.dims.km3_all * c->s.cfg.lm + 63) / 64;
+    return pick_tile(64 * chunks, c->nx[g], c->ny[g], c->b3H, false, true, 3072, 96).tj;
+}
+
 // Rows per wave of the radial pass over the 2-D variables (k >= K3) of
 // procedures 4 and 5: even, so that a restriction can ride in it. A few values
 // a column, a stack apart, are a cache line a lane: the lines a CU can ask for
@@ -913,7 +928,7 @@ int ball(mgbf_ctx* c, int g, const float* in, float* out, bool transpose, hipStr
         b.K3 = K3;
         b.H = c->b3H;
         b.HZ = c->b3HZ;
-        b.TJ = pick_tj(K3, b.n, b.m, 4);
+        b.TJ = ball3_tj(c, g);
         b.ball = c->b3ball;
         b.transpose = transpose ? 1 : 0;
         b.zero_levels = c->s.zero_levels ? 1 : 0;
@@ -1009,7 +1024,7 @@ int rad3_down(mgbf_ctx* c, const float* x, float* U, float* T, int g, bool* scal
     // the streaming pass loads at least 3 halo rows when it restricts
     // (so does the radial pass of the 2-D variables after K3)
     const bool res = next && c->ball3 && c->fuse >= 3 &&
-                     fused_ok(c, g, pick_tj(K3, c->nx[g], c->ny[g], 4), std::max(c->b3H, 3)) &&
+                     fused_ok(c, g, ball3_tj(c, g), std::max(c->b3H, 3)) &&
                      (K3 >= c->K || fused_ok(c, g, rad2d_tj(c, g), res_halo(c)));
     if (next && !res) CALL(restrict_g(c, g, ug, next, st));
     return ball(c, g, ug, T + c->goff[g], true, st, scaled, nullptr, res ? next : nullptr);
