@@ -250,8 +250,13 @@ int mgbf_timers_read_gen(mgbf_ctx* ctx, int gen, double* ms, long long* launches
    prolongation and the vertical band, 3 plain with the restriction to the
    next generation), and keeps the fastest. The candidate heights are a fixed
    ladder and the heights that fit the launch into whole rounds of the
-   chip's waves. For generation 1 it also times the vertical band as a pass
-   of its own after a kind-1 pass, and keeps that form when it beats kind 2.
+   chip's waves. Between the vector kernel and the matrix cores a near tie is
+   settled by rule, so that equal contexts tune to equal engines: at
+   half-widths of 6 and more a pass over 2^24 values or more goes to the matrix
+   cores up to 1.2 times the vector kernel's time, any other only below 0.95
+   times it. For generation 1 it
+   also times the vertical band as a pass of its own after a kind-1 pass, and
+   keeps that form when it beats kind 2.
    Uses the context's workspace; synchronizes `stream`. No counterpart in
    the reference, whose loops have no tiles. */
 int mgbf_autotune(mgbf_ctx* ctx, void* stream);
@@ -259,7 +264,9 @@ int mgbf_autotune(mgbf_ctx* ctx, void* stream);
    output columns per lane of the vector kernel (2 or 4), or 16 when the pass
    runs on the matrix cores (16 output columns x 64 k per block of 4
    wavefronts), or 0 for generation 1's kind 2 when the vertical band runs as
-   a pass of its own; *tj is the output rows per wavefront or block. */
+   a pass of its own; *tj is the output rows per wavefront or block. A pass
+   without a 2-column form (kind 2, and kind 1 of the quadratic transfer)
+   runs 4 columns per lane under ti = 2. */
 int mgbf_get_tile(const mgbf_ctx* ctx, int gen, int kind, int* ti, int* tj);
 /* Pins the tile of generation gen (1-based) and pass kind, in the terms of
    mgbf_get_tile (ti = 2 or 4, or 16 for the matrix cores, or 0 for
@@ -270,7 +277,9 @@ int mgbf_get_tile(const mgbf_ctx* ctx, int gen, int kind, int* ti, int* tj);
    multiple of 64 and a disc or product filter of half-width <= 8, with
    either transfer stencil (kind 2 also: half-width < 8; kind 3 also: at
    least 32 columns, half-width >= 3, exact FP16 restriction weights); else
-   MGBF_ERR_UNSUPPORTED. No counterpart in the reference. */
+   MGBF_ERR_UNSUPPORTED. The vector kernel carries the vertical band (kind 2)
+   up to half-width 8; wider filters run it as a pass of its own under any
+   tile. No counterpart in the reference. */
 int mgbf_set_tile(mgbf_ctx* ctx, int gen, int kind, int ti, int tj);
 
 /* Message of the last failure on this thread ("" if none). */

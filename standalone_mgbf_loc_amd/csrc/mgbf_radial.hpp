@@ -26,8 +26,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc_2g(const float* base)
 }
 
 // Row buffers of the input pipeline (one being combined, the others in
-// flight): 4 where the registers of the ring and its epilogues leave room.
-__host__ __device__ constexpr int radial_bufs(int H) { return H <= 6 ? 4 : (H <= 8 ? 3 : 2); }
+// flight): 4 where the registers of the ring and its epilogues leave room. A
+// narrow filter has too little arithmetic a row to be worth them: memory bounds
+// it on a large field, and more waves a SIMD use that better (the line procedure
+// at half-width 3, 80 x 768 x 768 x 64: 16.4 ms with 1 buffer, 16.8 with 2, 17.5
+// with 4 and the matrix cores beside; 1440 x 960 x 65 at half-width 1: 789, 798
+// and 801 us).
+__host__ __device__ constexpr int radial_bufs(int H) { return H <= 3 ? 1 : H <= 6 ? 4 : (H <= 8 ? 3 : 2); }
 
 // One step per ring row S, S+1, .. NR-1 of a turn; the first step past the
 // tile ends it (nested, so that no path rejoins another between two steps and
@@ -82,7 +87,8 @@ __device__ __forceinline__ void radial_turn(F& step, int rb, int nsteps) {
 // layout. The band takes stacks of whole 64-k chunks (with lm dividing 64 a
 // wave then holds whole columns).
 //
-// Input rows are loaded NB - 1 steps ahead into NB register buffers: the VALU
+// Input rows are loaded NB - 1 steps ahead into NB register buffers (none ahead
+// up to half-width 3, see radial_bufs): the VALU
 // is what bounds this kernel (62 operations an output for the H = 6 disc), and
 // with the loads in flight two waves a SIMD keep it 75-90 % busy. The ring has
 // the next multiple of NB above 2H rows, so that ring row and buffer of a step
