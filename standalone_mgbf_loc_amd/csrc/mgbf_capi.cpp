@@ -873,11 +873,13 @@ bool plan_ball3(const mgbf::Setup& s, const mgbf_config& cfg, mgbf::Ball3Coef& c
 // at 24, the least height for 16384 waves, the rule before; 384 x 384: 142 and
 // 129 at 48 (one round), 161 and 146 at 16. On 1536 x 1536 x 512 the waves of
 // 192 rows and more drift too far apart to share rows in the L2: an application
-// takes 9.03 ms at 96, 9.41 at 192, 9.98 at 24 (7.00, 7.39, 7.06 for the line
-// procedure).
+// takes 9.03 ms at 96, 9.41 at 192, 9.98 at 24. The line procedure's box has
+// less arithmetic to keep the waves together: 7.00, 7.39 and 7.06 ms there, and
+// with 4 two-dimensional variables behind (rows of 516 values, whose chunks
+// share cache lines) 11.13 at 96, 10.37 at 48, 9.76 at 24.
 int ball3_tj(const mgbf_ctx* c, int g) {
     const int chunks = (c->s.dims.km3_all * c->s.cfg.lm + 63) / 64;
-    return pick_tile(64 * chunks, c->nx[g], c->ny[g], c->b3H, false, true, 3072, 96).tj;
+    return pick_tile(64 * chunks, c->nx[g], c->ny[g], c->b3H, false, true, 3072, c->b3ball ? 96 : 24).tj;
 }
 
 // Rows per wave of the radial pass over the 2-D variables (k >= K3) of
