@@ -1180,36 +1180,38 @@ __global__ void __launch_bounds__(kBlock) aspect_kernel(AspectArgs a, int nkc, i
 // The rows of the transposed matrix from those of F: point p takes the weight
 // of every tap of p + g that reaches p, directly or through a mirror image of
 // p (the box holds all of them: folding moves a point towards the tap's
-// origin). One thread per weight.
+// origin). The threads stride over the weights: a launch of one thread each
+// would pass 2^32 threads, which HIP refuses, at 3120 x 3136 points of
+// half-width 10.
 __global__ void __launch_bounds__(kBlock) aspect_transpose_kernel(const float* __restrict__ w, float* __restrict__ wt,
                                                                 int n, int m, int H, long long count) {
-    const long long e = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (e >= count) return;
     const int NB = 2 * H + 1, nt = NB * NB;
-    const int t = (int)(e % nt);
-    const long long p = e / nt;
-    const int i = (int)(p % n), j = (int)(p / n);
-    const int sx = i + t % NB - H, sy = j + t / NB - H;
-    float acc = 0.f;
-    if (sx >= 0 && sx < n && sy >= 0 && sy < m) {
-        const float* ws = w + ((size_t)sx + (size_t)n * sy) * nt;
-        for (int b = 0; b < 3; ++b) {
-            const int gy = (b == 0 ? j : (b == 1 ? -1 - j : 2 * m - 1 - j)) - sy;
-            if (gy < -H || gy > H) continue;
-            for (int c = 0; c < 3; ++c) {
-                const int gx = (c == 0 ? i : (c == 1 ? -1 - i : 2 * n - 1 - i)) - sx;
-                if (gx >= -H && gx <= H) acc += ws[(gy + H) * NB + gx + H];
+    const long long stride = (long long)gridDim.x * kBlock;
+    for (long long e = (long long)blockIdx.x * kBlock + threadIdx.x; e < count; e += stride) {
+        const int t = (int)(e % nt);
+        const long long p = e / nt;
+        const int i = (int)(p % n), j = (int)(p / n);
+        const int sx = i + t % NB - H, sy = j + t / NB - H;
+        float acc = 0.f;
+        if (sx >= 0 && sx < n && sy >= 0 && sy < m) {
+            const float* ws = w + ((size_t)sx + (size_t)n * sy) * nt;
+            for (int b = 0; b < 3; ++b) {
+                const int gy = (b == 0 ? j : (b == 1 ? -1 - j : 2 * m - 1 - j)) - sy;
+                if (gy < -H || gy > H) continue;
+                for (int c = 0; c < 3; ++c) {
+                    const int gx = (c == 0 ? i : (c == 1 ? -1 - i : 2 * n - 1 - i)) - sx;
+                    if (gx >= -H && gx <= H) acc += ws[(gy + H) * NB + gx + H];
+                }
             }
         }
+        wt[e] = acc;
     }
-    wt[e] = acc;
 }
 
 hipError_t launch_aspect_transpose(const float* w, float* wt, int n, int m, int H, hipStream_t st) {
     const long long count = (long long)n * m * (2 * H + 1) * (2 * H + 1);
-    const long long nblocks = (count + kBlock - 1) / kBlock;
-    if (H < 1 || n < H || m < H || nblocks >= (1ll << 31)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(aspect_transpose_kernel, dim3((unsigned)nblocks), dim3(kBlock), 0, st, w, wt, n, m, H, count);
+    if (H < 1 || n < H || m < H) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(aspect_transpose_kernel, dim3(grid_for(count)), dim3(kBlock), 0, st, w, wt, n, m, H, count);
     return hipGetLastError();
 }
 
