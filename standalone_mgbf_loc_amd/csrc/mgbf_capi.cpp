@@ -97,6 +97,8 @@ struct mgbf_ctx {
     bool ball3 = false;
     mgbf::Ball3Coef b3{};
     int b3H = 0, b3HZ = 0, b3ball = 0;
+    // its rows per wave, and those of the radial pass over the 2-D variables
+    int ball3_tj[mgbf::kMaxGen] = {}, rad2d_tj[mgbf::kMaxGen] = {};
     const int4* d_t3 = nullptr;
     const float* d_w3 = nullptr;
     const int4* d_t2 = nullptr;
@@ -895,7 +897,7 @@ bool plan_ball3(const mgbf::Setup& s, const mgbf_config& cfg, mgbf::Ball3Coef& c
 // less arithmetic to keep the waves together: 7.00, 7.39 and 7.06 ms there, and
 // with 4 two-dimensional variables behind (rows of 516 values, whose chunks
 // share cache lines) 11.13 at 96, 10.37 at 48, 9.76 at 24.
-int ball3_tj(const mgbf_ctx* c, int g) {
+int pick_ball3_tj(const mgbf_ctx* c, int g) {
     const int chunks = (c->s.dims.km3_all * c->s.cfg.lm + 63) / 64;
     return pick_tile(64 * chunks, c->nx[g], c->ny[g], c->b3H, false, true, 3072, c->b3ball ? 96 : 24).tj;
 }
@@ -906,7 +908,7 @@ int ball3_tj(const mgbf_ctx* c, int g) {
 // bound the pass, not its VALU, and more than two waves a CU only repeat halo
 // rows (768 x 768 x 2 of 258: 57 us at 12 rows, 384 waves; 64 at 8 and at 16;
 // 91 at 4).
-int rad2d_tj(const mgbf_ctx* c, int g) {
+int pick_rad2d_tj(const mgbf_ctx* c, int g) {
     const int K3 = c->s.dims.km3_all * c->s.cfg.lm;
     return std::max(pick_tile(c->K - K3, c->nx[g], c->ny[g], c->s.H, false, true, 512).tj, std::min(c->ny[g], 4));
 }
@@ -948,7 +950,7 @@ int ball(mgbf_ctx* c, int g, const float* in, float* out, bool transpose, hipStr
         b.K3 = K3;
         b.H = c->b3H;
         b.HZ = c->b3HZ;
-        b.TJ = ball3_tj(c, g);
+        b.TJ = c->ball3_tj[g];
         b.ball = c->b3ball;
         b.transpose = transpose ? 1 : 0;
         b.zero_levels = c->s.zero_levels ? 1 : 0;
@@ -974,7 +976,7 @@ int ball(mgbf_ctx* c, int g, const float* in, float* out, bool transpose, hipStr
         r.m = c->ny[g];
         r.H = c->s.H;
         r.TI = 4;
-        r.TJ = rad2d_tj(c, g);
+        r.TJ = c->rad2d_tj[g];
         if (rout) {
             r.rout = rout;
             r.rytab = c->d_rytab[g];
@@ -1044,8 +1046,8 @@ int rad3_down(mgbf_ctx* c, const float* x, float* U, float* T, int g, bool* scal
     // the streaming pass loads at least 3 halo rows when it restricts
     // (so does the radial pass of the 2-D variables after K3)
     const bool res = next && c->ball3 && c->fuse >= 3 &&
-                     fused_ok(c, g, ball3_tj(c, g), std::max(c->b3H, 3)) &&
-                     (K3 >= c->K || fused_ok(c, g, rad2d_tj(c, g), res_halo(c)));
+                     fused_ok(c, g, c->ball3_tj[g], std::max(c->b3H, 3)) &&
+                     (K3 >= c->K || fused_ok(c, g, c->rad2d_tj[g], res_halo(c)));
     if (next && !res) CALL(restrict_g(c, g, ug, next, st));
     return ball(c, g, ug, T + c->goff[g], true, st, scaled, nullptr, res ? next : nullptr);
 }
@@ -1376,6 +1378,10 @@ int mgbf_init(const mgbf_config* cfg, int device, mgbf_ctx** out) {
             c->tile_ti[g][kind] = t.ti;
             c->tile_tj[g][kind] = t.tj;
             if (c->tile_mfma[g][kind]) c->tile_tj[g][kind] = pick_tj(c->K, s.nx[g], s.ny[g], 16);
+        }
+        if (c->ball3) {
+            c->ball3_tj[g] = pick_ball3_tj(c, g);
+            if (s.dims.km3_all * cfg->lm < c->K) c->rad2d_tj[g] = pick_rad2d_tj(c, g);
         }
         // the fused restriction needs an even number of rows per wave
         int& tj3 = c->tile_tj[g][3];
