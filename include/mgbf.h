@@ -264,9 +264,7 @@ int mgbf_autotune(mgbf_ctx* ctx, void* stream);
    output columns per lane of the vector kernel (2 or 4), or 16 when the pass
    runs on the matrix cores (16 output columns x 64 k per block of 4
    wavefronts), or 0 for generation 1's kind 2 when the vertical band runs as
-   a pass of its own; *tj is the output rows per wavefront or block. A pass
-   without a 2-column form (kind 2, and kind 1 of the quadratic transfer)
-   runs 4 columns per lane under ti = 2. */
+   a pass of its own; *tj is the output rows per wavefront or block. */
 int mgbf_get_tile(const mgbf_ctx* ctx, int gen, int kind, int* ti, int* tj);
 /* Pins the tile of generation gen (1-based) and pass kind, in the terms of
    mgbf_get_tile (ti = 2 or 4, or 16 for the matrix cores, or 0 for

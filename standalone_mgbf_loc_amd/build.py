@@ -95,7 +95,7 @@ def build(verbose: bool = False, jobs: int = 0) -> str:
         work.append((os.path.join(CSRC, BALL_TU), os.path.join(objdir, f"ball3_h{h}.o"),
                      [f"-DMGBF_BALL_H={h}"], verbose))
     for h in sorted(RADIAL_H, reverse=True):
-        for part in (1, 2, 0):
+        for part in (1, 2, 0, 3, 4):
             work.append((os.path.join(CSRC, RADIAL_TU), os.path.join(objdir, f"radial_h{h}_{part}.o"),
                          [f"-DMGBF_RADIAL_H={h}", f"-DMGBF_RADIAL_PART={part}"], verbose))
     jobs = jobs or min(len(work), max(1, (os.cpu_count() or 4)))

@@ -1928,9 +1928,7 @@ int mgbf_autotune(mgbf_ctx* c, void* stream) {
             const int engines[3] = {2, 4, 16};
             for (int en : engines) {
                 if (en == 16 && !try_mfma) continue;
-                // 2 columns a lane: the passes without a fused transfer, and
-                // the 4-point prolongation
-                if (en == 2 && (kind >= 2 || (kind == 1 && c->quad))) continue;
+                if (en == 2 && kind == 3) continue;   // the restriction takes 4 columns
                 // waves of one row of tiles (every column tile and k chunk)
                 const long long strip =
                     en == 16 ? (long long)(c->K / 64) * (n / 16) * 4 : mgbf::radial_row_waves(c->K, n, en);

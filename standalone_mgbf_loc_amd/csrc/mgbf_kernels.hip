@@ -535,11 +535,13 @@ hipError_t launch_radial(const RadialArgs& a, hipStream_t st) {
     // a k offset takes no band (whole columns are not in the wave) and no
     // matrix-core engine
     if (a.klo < 0 || a.klo >= a.K || (a.klo && (a.mfma || a.band))) return hipErrorInvalidValue;
-#define MGBF_RADIAL_CASE(h)                                   \
-    case h:                                                   \
-        if (a.mfma) return launch_radial_mx_H##h(a, st);      \
-        if (a.exact_disc) return launch_radial_disc_H##h(a, st); \
-        return a.separable ? launch_radial_sep_H##h(a, st) : launch_radial_box_H##h(a, st);
+    const bool two = a.TI == 2 && !a.rout;
+#define MGBF_RADIAL_CASE(h)                                                                       \
+    case h:                                                                                       \
+        if (a.mfma) return launch_radial_mx_H##h(a, st);                                          \
+        if (a.exact_disc) return two ? launch_radial_disc2_H##h(a, st) : launch_radial_disc_H##h(a, st); \
+        if (a.separable) return two ? launch_radial_sep2_H##h(a, st) : launch_radial_sep_H##h(a, st);   \
+        return two ? launch_radial_box2_H##h(a, st) : launch_radial_box_H##h(a, st);
     switch (a.H) {
         MGBF_RADIAL_CASE(1) MGBF_RADIAL_CASE(2) MGBF_RADIAL_CASE(3) MGBF_RADIAL_CASE(4) MGBF_RADIAL_CASE(5)
         MGBF_RADIAL_CASE(6) MGBF_RADIAL_CASE(7) MGBF_RADIAL_CASE(8) MGBF_RADIAL_CASE(9) MGBF_RADIAL_CASE(10)

@@ -47,7 +47,7 @@ struct RadialArgs {
     int klo;              // first k filtered (k < klo is left alone): 0, or K3 for
                           // the 2-D variables after the 3-D ones of procedures 4, 5
     int H;                // max(hx, hy)
-    int TI;               // output columns per lane (2 or 4; 2 runs as 4 where it is not built)
+    int TI;               // output columns per lane (2, or 4; 4 with rout)
     // matrix-core engine (mgbf_radial_mx.hpp)
     bool mfma;
     const void* bfrag;      // FP16 hi/lo B fragments of the Toeplitz weight bands T_b
@@ -127,7 +127,10 @@ constexpr long long radial_row_waves(int kc, int n, int TI) {
     hipError_t launch_radial_mx_H##h(const RadialArgs& a, hipStream_t st);    \
     hipError_t launch_radial_box_H##h(const RadialArgs& a, hipStream_t st);   \
     hipError_t launch_radial_disc_H##h(const RadialArgs& a, hipStream_t st);  \
-    hipError_t launch_radial_sep_H##h(const RadialArgs& a, hipStream_t st);
+    hipError_t launch_radial_sep_H##h(const RadialArgs& a, hipStream_t st);   \
+    hipError_t launch_radial_box2_H##h(const RadialArgs& a, hipStream_t st);  \
+    hipError_t launch_radial_disc2_H##h(const RadialArgs& a, hipStream_t st); \
+    hipError_t launch_radial_sep2_H##h(const RadialArgs& a, hipStream_t st);
 MGBF_DECLARE_RADIAL(1) MGBF_DECLARE_RADIAL(2) MGBF_DECLARE_RADIAL(3) MGBF_DECLARE_RADIAL(4)
 MGBF_DECLARE_RADIAL(5) MGBF_DECLARE_RADIAL(6) MGBF_DECLARE_RADIAL(7) MGBF_DECLARE_RADIAL(8)
 MGBF_DECLARE_RADIAL(9) MGBF_DECLARE_RADIAL(10)

@@ -505,38 +505,48 @@ hipError_t launch_radial_variant(const RadialArgs& a, hipStream_t st) {
 }
 
 // The pass kinds; radial_built, checked here, lists what is built.
-template <int H, int TAPS, int VHB>
+template <int H, int TI, int TAPS, int VHB>
 hipError_t launch_radial_band(const RadialArgs& a, hipStream_t st) {
     if constexpr (H <= kVecMaxBandH && TAPS != kTapsBox)
-        return a.quad ? launch_radial_variant<H, 4, TAPS, true, VHB, false, true>(a, st)
-                      : launch_radial_variant<H, 4, TAPS, true, VHB, false, false>(a, st);
+        return a.quad ? launch_radial_variant<H, TI, TAPS, true, VHB, false, true>(a, st)
+                      : launch_radial_variant<H, TI, TAPS, true, VHB, false, false>(a, st);
     else
         return hipErrorInvalidValue;
 }
 
+template <int H, int TI, int TAPS>
+hipError_t launch_radial_ti(const RadialArgs& a, hipStream_t st) {
+    if (a.band) {
+        switch (a.vhb) {
+            case 3: return launch_radial_band<H, TI, TAPS, 3>(a, st);
+            case 4: return launch_radial_band<H, TI, TAPS, 4>(a, st);
+            case 6: return launch_radial_band<H, TI, TAPS, 6>(a, st);
+            case 8: return launch_radial_band<H, TI, TAPS, 8>(a, st);
+            default: return hipErrorInvalidValue;
+        }
+    }
+    if (!a.coarse) return launch_radial_variant<H, TI, TAPS, false, 0, false, false>(a, st);
+    return a.quad ? launch_radial_variant<H, TI, TAPS, true, 0, false, true>(a, st)
+                  : launch_radial_variant<H, TI, TAPS, true, 0, false, false>(a, st);
+}
+
+// Passes of 4 columns a lane, and those with the restriction
 template <int H, int TAPS>
 hipError_t launch_radial_taps(const RadialArgs& a, hipStream_t st) {
     if (!radial_built(a) || a.TJ < 1 || (TAPS == kTapsDisc) != a.exact_disc || (TAPS == kTapsSep) != a.separable)
         return hipErrorInvalidValue;
-    if (a.band) {
-        switch (a.vhb) {
-            case 3: return launch_radial_band<H, TAPS, 3>(a, st);
-            case 4: return launch_radial_band<H, TAPS, 4>(a, st);
-            case 6: return launch_radial_band<H, TAPS, 6>(a, st);
-            case 8: return launch_radial_band<H, TAPS, 8>(a, st);
-            default: return hipErrorInvalidValue;
-        }
-    }
     if (a.rout)
         return a.quad ? launch_radial_variant<H, 4, TAPS, false, 0, true, true>(a, st)
                       : launch_radial_variant<H, 4, TAPS, false, 0, true, false>(a, st);
-    if constexpr (TAPS != kTapsBox) {   // 2 columns a lane, for the smallest launches
-        if (a.TI == 2 && !a.coarse) return launch_radial_variant<H, 2, TAPS, false, 0, false, false>(a, st);
-        if (a.TI == 2 && !a.quad) return launch_radial_variant<H, 2, TAPS, true, 0, false, false>(a, st);
-    }
-    if (!a.coarse) return launch_radial_variant<H, 4, TAPS, false, 0, false, false>(a, st);
-    return a.quad ? launch_radial_variant<H, 4, TAPS, true, 0, false, true>(a, st)
-                  : launch_radial_variant<H, 4, TAPS, true, 0, false, false>(a, st);
+    return launch_radial_ti<H, 4, TAPS>(a, st);
+}
+
+// Passes of 2 columns a lane
+template <int H, int TAPS>
+hipError_t launch_radial_taps2(const RadialArgs& a, hipStream_t st) {
+    if (!radial_built(a) || a.rout || a.TJ < 1 || (TAPS == kTapsDisc) != a.exact_disc || (TAPS == kTapsSep) != a.separable)
+        return hipErrorInvalidValue;
+    return launch_radial_ti<H, 2, TAPS>(a, st);
 }
 
 }  // namespace mgbf
