@@ -275,9 +275,7 @@ int mgbf_get_tile(const mgbf_ctx* ctx, int gen, int kind, int* ti, int* tj);
    multiple of 64 and a disc or product filter of half-width <= 8, with
    either transfer stencil (kind 2 also: half-width < 8; kind 3 also: at
    least 32 columns, half-width >= 3, exact FP16 restriction weights); else
-   MGBF_ERR_UNSUPPORTED. The vector kernel carries the vertical band (kind 2)
-   up to half-width 8; wider filters run it as a pass of its own under any
-   tile. No counterpart in the reference. */
+   MGBF_ERR_UNSUPPORTED. No counterpart in the reference. */
 int mgbf_set_tile(mgbf_ctx* ctx, int gen, int kind, int ti, int tj);
 
 /* Message of the last failure on this thread ("" if none). */

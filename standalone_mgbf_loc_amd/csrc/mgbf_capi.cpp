@@ -458,7 +458,7 @@ bool can_fuse_band(const mgbf_ctx* c, int which) {
     const int hb = c->band_hb[which];
     const int lm = c->s.cfg.lm;
     return c->nfilt > 0 && (c->s.exact_disc || c->s.separable) && c->gm > 1 && (64 % lm) == 0 &&
-           (c->K % 64) == 0 && c->s.H <= mgbf::kVecMaxBandH &&
+           (c->K % 64) == 0 &&
            (hb == 3 || hb == 4 || hb == 6 || hb == 8);
 }
 

@@ -528,7 +528,7 @@ bool radial_built(const RadialArgs& a) {
     if (a.TI != 2 && a.TI != 4) return false;
     if (!a.band) return true;
     const bool hb = a.vhb == 3 || a.vhb == 4 || a.vhb == 6 || a.vhb == 8;
-    return hb && (a.exact_disc || a.separable) && a.coarse && !a.klo && a.H <= kVecMaxBandH && a.lm >= 1 && kWave % a.lm == 0 && a.K % kWave == 0;
+    return hb && (a.exact_disc || a.separable) && a.coarse && !a.klo && a.lm >= 1 && kWave % a.lm == 0 && a.K % kWave == 0;
 }
 
 hipError_t launch_radial(const RadialArgs& a, hipStream_t st) {

@@ -106,9 +106,6 @@ struct RadialMxParams {
     int ntile_i, ntile_j;
 };
 
-// the vector kernel takes the vertical band up to this half-width (beyond it
-// the band's registers do not fit beside the ring and the row buffers)
-constexpr int kVecMaxBandH = 8;
 // Is the vector kernel built for this pass (its taps, epilogues and stack)?
 bool radial_built(const RadialArgs& a);
 // The vector kernel lays the kc stacked values of a tile row's column tiles

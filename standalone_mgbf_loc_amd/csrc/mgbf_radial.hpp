@@ -32,7 +32,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc_2g(const float* base)
 // at half-width 3, 80 x 768 x 768 x 64: 16.4 ms with 1 buffer, 16.8 with 2, 17.5
 // with 4 and the matrix cores beside; 1440 x 960 x 65 at half-width 1: 789, 798
 // and 801 us).
-__host__ __device__ constexpr int radial_bufs(int H) { return H <= 3 ? 1 : H <= 6 ? 4 : (H <= 8 ? 3 : 2); }
+// With the band beside 4 columns, the disc of half-width 10 has registers for one
+// only (256 registers and one wave a SIMD with 2: 512 x 512 x 1024, whole
+// application, 4.29 ms against 3.73).
+__host__ __device__ constexpr int radial_bufs(int H, int TI, bool disc, int VHB) {
+    if (H > 9 && TI == 4 && disc && VHB > 0) return 1;
+    return H <= 3 ? 1 : H <= 6 ? 4 : (H <= 8 ? 3 : 2);
+}
 
 // One step per ring row S, S+1, .. NR-1 of a turn; the first step past the
 // tile ends it (nested, so that no path rejoins another between two steps and
@@ -109,7 +115,7 @@ __global__ void __launch_bounds__(kBlock) radial_kernel(RadialParams p) {
     static_assert(!QP || PRO || (RES && VHB == 0), "the quadratic transfer rides in PRO or RES");
     static_assert(!RES || (TI == 4 && !PRO && VHB == 0), "restriction epilogue shape");
     constexpr bool DISC = TAPS == kTapsDisc;
-    constexpr int NB = radial_bufs(H);
+    constexpr int NB = radial_bufs(H, TI, DISC, VHB);
     constexpr int NR = (2 * H + 1 + NB - 1) / NB * NB;
     // columns and rows loaded on each side: H for the filter, 4 columns and 3
     // rows for the restriction's 8-point stencils; the D extra rows feed the
@@ -507,7 +513,7 @@ hipError_t launch_radial_variant(const RadialArgs& a, hipStream_t st) {
 // The pass kinds; radial_built, checked here, lists what is built.
 template <int H, int TI, int TAPS, int VHB>
 hipError_t launch_radial_band(const RadialArgs& a, hipStream_t st) {
-    if constexpr (H <= kVecMaxBandH && TAPS != kTapsBox)
+    if constexpr (TAPS != kTapsBox)
         return a.quad ? launch_radial_variant<H, TI, TAPS, true, VHB, false, true>(a, st)
                       : launch_radial_variant<H, TI, TAPS, true, VHB, false, false>(a, st);
     else
