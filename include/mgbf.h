@@ -248,15 +248,16 @@ int mgbf_timers_read_gen(mgbf_ctx* ctx, int gen, double* ms, long long* launches
    (output columns per lane x output rows per wavefront), for each generation
    and each pass kind (0 plain, 1 with the prolongation, 2 with the
    prolongation and the vertical band, 3 plain with the restriction to the
-   next generation), and keeps the fastest. The candidate heights are a fixed
-   ladder and the heights that fit the launch into whole rounds of the
-   chip's waves. Between the vector kernel and the matrix cores a near tie is
-   settled by rule, so that equal contexts tune to equal engines: at
-   half-widths of 6 and more a pass over 2^24 values or more goes to the matrix
-   cores up to 1.2 times the vector kernel's time, any other only below 0.95
-   times it. For generation 1 it
-   also times the vertical band as a pass of its own after a kind-1 pass, and
-   keeps that form when it beats kind 2.
+   next generation), and keeps the fastest tile of each engine. The candidate
+   heights are a fixed ladder and the heights that fit the launch into whole
+   rounds of the chip's waves. Between the vector kernel and the matrix cores,
+   whose results differ in rounding, a rule chooses: at half-widths of 6 and
+   more a pass over 2^24 values or more goes to the matrix cores up to 1.2
+   times the vector kernel's time, any other only below 0.95 times it. So the
+   engine kept may be slower by up to a fifth, and equal contexts mostly, but
+   not always, tune to equal engines: mgbf_set_tile pins what one run found.
+   For generation 1 it also times the vertical band as a pass of its own after
+   a kind-1 pass, and keeps that form when it beats kind 2.
    Uses the context's workspace; synchronizes `stream`. No counterpart in
    the reference, whose loops have no tiles. */
 int mgbf_autotune(mgbf_ctx* ctx, void* stream);

@@ -1979,15 +1979,20 @@ int mgbf_autotune(mgbf_ctx* c, void* stream) {
                     }
                 }
             }
-            // a near tie is not left to the noise of three timed passes, which
-            // would choose the engine, and with it the rounding, anew in every
-            // run: with a wide filter a pass over 2^24 values or more goes to
-            // the matrix cores unless they take 1.2x the time. A smaller one
-            // (whose 16-column tiles are the scarcer, the smaller it is) goes
-            // there only if they take less than 0.95x, and so does one of a
-            // narrow filter, which both engines do at the memory's rate on the
-            // zeros timed here, but not on data (the line procedure on 80 x
-            // 768 x 768 x 64: 16.2 ms, 17.5 with the ties on the matrix cores)
+            // the engine decides the rounding, so that the choice is kept off
+            // the ratio of 1, where the noise of three timed passes would make
+            // it anew in every run: with a wide filter a pass over 2^24 values
+            // or more goes to the matrix cores unless they take 1.2x the time.
+            // That gives up 2 to 14 % of a pass (9 to 19 % on data) in the third
+            // generation of 512 x 512 x 1024 at half-width 6, under 1 % of an
+            // application; the larger passes are faster there by 3 to 18 %. A
+            // smaller one (whose
+            // 16-column tiles are the scarcer, the smaller it is) goes there
+            // only if they take less than 0.95x, and so does one of a narrow
+            // filter, which both engines do at the memory's rate on the zeros
+            // timed here, but not on data (the line procedure on 80 x 768 x 768
+            // x 64: 16.2 ms, 17.5 with the ties on the matrix cores). Near 1.2
+            // and 0.95 the choice is as open as it would be near 1
             const double tie = c->s.H >= 6 && (double)c->K * n * m >= 16777216.0 ? 1.2 : 0.95;
             const bool mx = bestm < 1e30f && bestm <= tie * best;
             c->tile_ti[g][kind] = mx ? 4 : bti;

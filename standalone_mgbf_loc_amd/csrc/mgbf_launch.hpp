@@ -109,8 +109,8 @@ struct RadialMxParams {
 // Is the vector kernel built for this pass (its taps, epilogues and stack)?
 bool radial_built(const RadialArgs& a);
 // The vector kernel lays the kc stacked values of a tile row's column tiles
-// end to end where chunks of 64 k would idle an eighth of the lanes or more
-// (kc = 32, 65, 130, 2): below that the chunks' order, tiles fastest, reads
+// end to end where chunks of 64 k would idle a ninth of the lanes or more
+// (kc = 32, 65, 113, 130, 2): below that the chunks' order, tiles fastest, reads
 // memory in longer runs (512 x 512 x 520, generation 3: 38 us against 42 us
 // end to end, for 3.4 % idle lanes).
 constexpr bool radial_flattened(int kc) { return kc % 64 && 64ll * ((kc + 63) / 64) * 8 >= 9ll * kc; }

@@ -96,7 +96,10 @@ __device__ __forceinline__ void radial_turn(F& step, int rb, int nsteps) {
 // Input rows are loaded NB - 1 steps ahead into NB register buffers (none ahead
 // up to half-width 3, see radial_bufs): the VALU
 // is what bounds this kernel (62 operations an output for the H = 6 disc), and
-// with the loads in flight two waves a SIMD keep it 75-90 % busy. The ring has
+// with the loads in flight two waves a SIMD keep it busy: 89 % (with RES) and all
+// of the time (PRO and the band) on 768 x 768 x 5120, 66 and 79 % in the one round
+// of 384 x 384 x 320; at H = 8 on 1024 x 1024 x 127, 63 % (RES) and 79 % (PRO); at
+// H = 1, where memory bounds it, 21 and 23 %. The ring has
 // the next multiple of NB above 2H rows, so that ring row and buffer of a step
 // are compile-time constants; the spare rows cost TI registers each.
 // 512 x 512 x 1024 at H = 6: 0.54 ms plain, 0.60 with PRO, 0.70 with PRO and

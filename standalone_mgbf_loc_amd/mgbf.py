@@ -464,7 +464,11 @@ class MGBF:
 
     def autotune(self, stream=None) -> dict:
         """Times the candidate radial tiles on this context's shapes and keeps
-        the fastest; returns {(gen, kind): (TI, TJ)}. TI = 0 for (1, 2): the
+        the fastest of each engine, and of the engines the one that
+        mgbf_autotune's rule prefers (the matrix cores on large passes of wide
+        filters up to 1.2 times the vector kernel's time); returns
+        {(gen, kind): (TI, TJ)}. Equal contexts mostly, but not always, tune to
+        equal engines: set_tiles pins them. TI = 0 for (1, 2): the
         vertical band runs as a pass of its own after the kind-1 pass, which
         was faster than the band fused into it."""
         _check(self._L.mgbf_autotune(self._h, _stream(stream)))
