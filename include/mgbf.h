@@ -172,9 +172,10 @@ int mgbf_set_weights(mgbf_ctx* ctx, int gen, const float* field, double value);
    ellipse and normalizer, and F^T (no longer F) is the transposed gather of
    the scatter and fold. Built for the radial procedures 1 and 6
    (MGBF_ERR_UNSUPPORTED otherwise); a reach beyond the halo is refused with
-   the reference's message. The weights of each point's taps, for F and for
-   F^T, are kept on the device: 2 (2H+1)^2 floats per point of the
-   generation. */
+   the reference's message. The weights of each point's taps are kept on the
+   device, (2H+1)^2 floats per point of the generation, and as many for F^T if
+   there is room for them; without them (or with MGBF_ASPECT_SCATTER=1 in the
+   environment of mgbf_init) F^T takes about 20 times as long. */
 int mgbf_set_aspect(mgbf_ctx* ctx, int gen, const double* pasp2);
 
 /* Applies an operator (MGBF_OP_*). For WAWT, `in` and `out` may alias. The

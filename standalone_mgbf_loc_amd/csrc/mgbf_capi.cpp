@@ -141,9 +141,11 @@ struct mgbf_ctx {
     const float* wfield[mgbf::kMaxGen] = {};
     float wconst[mgbf::kMaxGen] = {};
     // per-point aspect tensors (mgbf_set_aspect): the weights of every
-    // point's taps over the (2H+1)^2 box, then the same of F^T, which is a
-    // filter of its own
+    // point's taps over the (2H+1)^2 box, and the same of F^T, which is a
+    // filter of its own (nullptr: F^T goes by the taps of F)
     float* d_aw[mgbf::kMaxGen] = {};
+    float* d_awt[mgbf::kMaxGen] = {};
+    bool aspect_scatter = false;   // MGBF_ASPECT_SCATTER=1: no rows of F^T
     bool aniso[mgbf::kMaxGen] = {};
     // analysis <-> filter transfer: separable window tables (direct: filter ->
     // analysis, adjoint: its transpose) and the vertical k windows
@@ -485,13 +487,12 @@ int radial(mgbf_ctx* c, int g, const float* in, float* out, const float* wfield,
         // or band epilogue rides in it
         if (coarse || rout || band >= 0)
             return fail(MGBF_ERR_ARG, "internal: epilogue fused into a per-point aspect pass");
-        const float* aw = c->d_aw[g];
-        if (transpose) {
-            const size_t nb = 2 * (size_t)c->s.H + 1;
-            aw += (size_t)c->nx[g] * c->ny[g] * nb * nb;
-        }
+        const float* aw = transpose && c->d_awt[g] ? c->d_awt[g] : c->d_aw[g];
         mgbf::AspectArgs aa{in, out, aw, c->K, c->nx[g], c->ny[g], c->s.H, wfield, wconst};
-        HIP_TRY(mgbf::launch_aspect(aa, transpose, st), "aspect filter launch");
+        if (transpose && !c->d_awt[g])
+            HIP_TRY(mgbf::launch_aspect_scatter(aa, st), "aspect filter launch");
+        else
+            HIP_TRY(mgbf::launch_aspect(aa, transpose, st), "aspect filter launch");
         return MGBF_OK;
     }
     mgbf::RadialArgs a{};
@@ -1342,6 +1343,9 @@ int mgbf_init(const mgbf_config* cfg, int device, mgbf_ctx** out) {
     {
         const char* xg = std::getenv("MGBF_XFER_GATHER");
         c->xfer_gather = xg && xg[0] == '1';
+        // MGBF_ASPECT_SCATTER=1 keeps the aspect weights of F alone (half the memory)
+        const char* as = std::getenv("MGBF_ASPECT_SCATTER");
+        c->aspect_scatter = as && as[0] == '1';
         const char* xs = std::getenv("MGBF_XFER_SPLIT");
         c->xfer_split = xs && xs[0] == '1';
     }
@@ -1726,7 +1730,8 @@ int mgbf_finalize(mgbf_ctx* c) {
     if (c->d_tables) (void)hipFree(c->d_tables);
     if (c->ws_a) (void)hipFree(c->ws_a);
     for (int g = 0; g < mgbf::kMaxGen; ++g)
-        if (c->d_aw[g]) (void)hipFree(c->d_aw[g]);
+        for (float* p : {c->d_aw[g], c->d_awt[g]})
+            if (p) (void)hipFree(p);
     delete c;
     return MGBF_OK;
 }
@@ -1755,8 +1760,9 @@ int mgbf_set_aspect(mgbf_ctx* c, int gen, const double* pasp2) {
         if (c->d_aw[g]) {
             HIP_TRY(hipDeviceSynchronize(), "synchronize before freeing the aspect weights");
             HIP_TRY(hipFree(c->d_aw[g]), "hipFree(aspect weights)");
+            if (c->d_awt[g]) HIP_TRY(hipFree(c->d_awt[g]), "hipFree(aspect weights)");
         }
-        c->d_aw[g] = nullptr;
+        c->d_aw[g] = c->d_awt[g] = nullptr;
         c->aniso[g] = false;
         ++c->version;
         return MGBF_OK;
@@ -1769,12 +1775,17 @@ int mgbf_set_aspect(mgbf_ctx* c, int gen, const double* pasp2) {
     std::string err;
     const int st = mgbf::aspect_weights(c->s.cfg, c->s.H, c->nx[g], c->ny[g], pasp2, w, &err);
     if (st != MGBF_OK) return fail(st, err);
-    // the taps of F, and behind them the rows of the transposed matrix
-    if (!c->d_aw[g]) HIP_TRY(hipMalloc(&c->d_aw[g], 2 * sizeof(float) * w.size()), "hipMalloc(aspect weights)");
+    // the taps of F, and the rows of the transposed matrix if there is room
+    if (!c->d_aw[g]) HIP_TRY(hipMalloc(&c->d_aw[g], sizeof(float) * w.size()), "hipMalloc(aspect weights)");
+    if (!c->d_awt[g] && !c->aspect_scatter && hipMalloc(&c->d_awt[g], sizeof(float) * w.size()) != hipSuccess) {
+        c->d_awt[g] = nullptr;
+        (void)hipGetLastError();
+    }
     HIP_TRY(hipMemcpy(c->d_aw[g], w.data(), sizeof(float) * w.size(), hipMemcpyHostToDevice),
             "aspect weights upload");
-    HIP_TRY(mgbf::launch_aspect_transpose(c->d_aw[g], c->d_aw[g] + w.size(), c->nx[g], c->ny[g], c->s.H, nullptr),
-            "aspect weights transposition");
+    if (c->d_awt[g])
+        HIP_TRY(mgbf::launch_aspect_transpose(c->d_aw[g], c->d_awt[g], c->nx[g], c->ny[g], c->s.H, nullptr),
+                "aspect weights transposition");
     // a later apply may run on a stream that does not wait for this one
     HIP_TRY(hipStreamSynchronize(nullptr), "aspect weights transposition");
     c->aniso[g] = true;

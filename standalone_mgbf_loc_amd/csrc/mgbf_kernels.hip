@@ -12,6 +12,7 @@
 // uses precomputed transposed tables.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 #include "mgbf_device.hpp"
@@ -1214,6 +1215,55 @@ hipError_t launch_aspect_transpose(const float* w, float* wt, int n, int m, int 
     const long long count = (long long)n * m * (2 * H + 1) * (2 * H + 1);
     if (H < 1 || n < H || m < H) return hipErrorInvalidValue;
     hipLaunchKernelGGL(aspect_transpose_kernel, dim3(grid_for(count)), dim3(kBlock), 0, st, w, wt, n, m, H, count);
+    return hipGetLastError();
+}
+
+// F^T without the rows of the transposed matrix, for a device that has no room
+// for them: one wave per point and 64 k collects, over the mirror preimages e of
+// the point (per axis -1-q within H of the low edge, 2n-1-q within H of the high
+// one) and the taps t whose source e - g_t lies in the domain, that source's
+// weight times its value. Each tap is a scalar load, a branch and a vector load:
+// 850 us on 256 x 256 x 64 at H = 6, where the rows take 37.
+__global__ void __launch_bounds__(kBlock) aspect_scatter_kernel(AspectArgs a) {
+    const int H = a.H, NB = 2 * H + 1, n = a.n, m = a.m;
+    const size_t K = (size_t)a.K;
+    const int k = blockIdx.y * kWave + (threadIdx.x & (kWave - 1));
+    const bool kvalid = k < a.K;
+    const int kk = kvalid ? k : a.K - 1;
+    const long long npts = (long long)n * m;
+    for (long long pt = (long long)blockIdx.x * kWavesPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+         pt < npts; pt += (long long)gridDim.x * kWavesPerBlock) {
+        const int i = (int)(pt % n), j = (int)(pt / n);
+        float acc = 0.f;
+        for (int b = 0; b < 3; ++b) {
+            if ((b == 1 && j > H - 1) || (b == 2 && j < m - H)) continue;
+            const int ey = b == 0 ? j : (b == 1 ? -1 - j : 2 * m - 1 - j);
+            for (int gy = -H; gy <= H; ++gy) {
+                const int sy = ey - gy;
+                if (sy < 0 || sy >= m) continue;
+                for (int c = 0; c < 3; ++c) {
+                    if ((c == 1 && i > H - 1) || (c == 2 && i < n - H)) continue;
+                    const int ex = c == 0 ? i : (c == 1 ? -1 - i : 2 * n - 1 - i);
+                    for (int gx = -H; gx <= H; ++gx) {
+                        const int sx = ex - gx;
+                        if (sx < 0 || sx >= n) continue;
+                        const size_t sp = (size_t)sx + (size_t)n * sy;
+                        const float wv = a.w[sp * NB * NB + (gy + H) * NB + gx + H];
+                        if (wv != 0.f) acc = __builtin_fmaf(wv, a.in[kk + K * sp], acc);
+                    }
+                }
+            }
+        }
+        const size_t o = kk + K * (size_t)pt;
+        if (kvalid) a.out[o] = (a.wfield ? a.wfield[o] : a.wconst) * acc;
+    }
+}
+
+hipError_t launch_aspect_scatter(const AspectArgs& a, hipStream_t st) {
+    if (a.H < 1 || a.n < a.H || a.m < a.H || a.K < 1) return hipErrorInvalidValue;
+    const long long nkc = (a.K + kWave - 1) / kWave, nb = ((long long)a.n * a.m + kWavesPerBlock - 1) / kWavesPerBlock;
+    if (nkc > 65535) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(aspect_scatter_kernel, dim3((unsigned)std::min(nb, 1ll << 20), (unsigned)nkc), dim3(kBlock), 0, st, a);
     return hipGetLastError();
 }
 

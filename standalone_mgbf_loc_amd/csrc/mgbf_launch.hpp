@@ -174,6 +174,8 @@ struct AspectArgs {
     float wconst;         // constant scale when wfield is nullptr
 };
 hipError_t launch_aspect(const AspectArgs& a, bool transpose, hipStream_t st);
+// F^T from the taps w of F (no rows of the transposed matrix)
+hipError_t launch_aspect_scatter(const AspectArgs& a, hipStream_t st);
 // wt = the rows of the transposed matrix, from the taps w of F
 hipError_t launch_aspect_transpose(const float* w, float* wt, int n, int m, int H, hipStream_t st);
 
