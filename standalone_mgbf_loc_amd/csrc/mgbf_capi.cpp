@@ -299,16 +299,12 @@ Tile pick_tile(int kc, int n, int m, int H, bool two, bool even, long long slots
 // that share halo rows drift too far apart for the L2. The line procedure's
 // application at half-width 3 on 512 x 512 x 1024: 1.92 ms at whole columns
 // (one round of 2048 waves), 1.46 at up to 86 rows, 1.47 at 48, 1.73 at 8; on
-// 768 x 768 x 64 329 us at 77 rows (1920 waves), 256 at 37. Rows below 24 (16 in
-// a plain pass) are not worth the second two of the 4 waves: 304 x 296 x 127, 147
-// us at 12, 144 at 23 (one round of 2048); the plain pass on 192 x 960 x 64 19 us
-// at 16 and at 12, 22 at 23.
+// 768 x 768 x 64 329 us at 77 rows (1920 waves), 256 at 37; on 192 x 960 x 64
+// 113 at 23 (2016 waves), 102 at 12.
 Tile default_tile(int K, int n, int m, int H, int kind) {
     const bool even = kind == 3;
     const Tile t = pick_tile(K, n, m, H, kind < 2, even);
-    if (H > 3 || t.ti != 4) return t;
-    const Tile u = pick_tile(K, n, m, H, false, even, 4096, 96);
-    return {4, std::max(u.tj, std::min(t.tj, kind == 0 ? 16 : 24))};
+    return H > 3 || t.ti != 4 ? t : pick_tile(K, n, m, H, false, even, 4096, 96);
 }
 
 enum { BAND_VF = 0, BAND_VFT = 1, BAND_VVT = 2 };
