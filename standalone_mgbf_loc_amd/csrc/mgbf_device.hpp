@@ -29,13 +29,11 @@ __device__ __forceinline__ int mirror_whole(int q, int n) {
 }
 
 // Blocks are dispatched round-robin over the 8 XCDs; give each XCD a
-// contiguous range of logical blocks so neighbouring tiles share its L2. XCD x
-// takes the blocks x, x + 8, ..: one more than nblocks / 8 for the first
-// nblocks % 8 of them.
+// contiguous range of logical blocks so neighbouring tiles share its L2.
 __device__ __forceinline__ unsigned xcd_block(unsigned bid, unsigned nblocks) {
     constexpr unsigned kXcd = 8;
-    const unsigned x = bid % kXcd, r = nblocks % kXcd;
-    return x * (nblocks / kXcd) + (x < r ? x : r) + bid / kXcd;
+    if (nblocks % kXcd) return bid;
+    return (bid % kXcd) * (nblocks / kXcd) + bid / kXcd;
 }
 
 // Buffer resource over 4 GiB from `base`: raw dword accesses address
