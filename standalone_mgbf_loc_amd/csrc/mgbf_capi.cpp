@@ -295,16 +295,21 @@ Tile pick_tile(int kc, int n, int m, int H, bool two, bool even, long long slots
 
 // Default tile of a generation's radial passes. Up to half-width 3 there is too
 // little arithmetic a row to hide the loads behind, or to keep the waves
-// together: 4 waves a SIMD instead of 2, and at most 96 rows, past which waves
-// that share halo rows drift too far apart for the L2. The line procedure's
-// application at half-width 3 on 512 x 512 x 1024: 1.92 ms at whole columns
-// (one round of 2048 waves), 1.46 at up to 86 rows, 1.47 at 48, 1.73 at 8; on
-// 768 x 768 x 64 329 us at 77 rows (1920 waves), 256 at 37; on 192 x 960 x 64
-// 113 at 23 (2016 waves), 102 at 12.
+// together, so that heights over 32 rows give way to 4 waves a SIMD instead of
+// 2 and at most 96 rows, past which waves that share halo rows drift too far
+// apart for the L2. The line procedure's application at half-width 3 on 512 x
+// 512 x 1024: 1.92 ms at whole columns (one round of 2048 waves), 1.46 at up to
+// 86 rows, 1.47 at 48, 1.73 at 8; on 768 x 768 x 64 329 us at 77 rows (1920
+// waves), 256 at 37. From lower heights more waves gain nothing (the fast filter
+// on 304 x 216 x 704, 277 us at 32 rows, 292 at 24), nor on stacks that are not
+// whole 64-k chunks, whose neighbouring waves share cache lines (on 136 x 752 x
+// 1905, 1.79 ms at 376 rows, 2.22 at 94; on 112 x 592 x 195 162 us at 26, 171 at
+// 16).
 Tile default_tile(int K, int n, int m, int H, int kind) {
     const bool even = kind == 3;
     const Tile t = pick_tile(K, n, m, H, kind < 2, even);
-    return H > 3 || t.ti != 4 ? t : pick_tile(K, n, m, H, false, even, 4096, 96);
+    if (H > 3 || K % 64 || t.tj <= 32) return t;
+    return {4, std::max(pick_tile(K, n, m, H, false, even, 4096, 96).tj, 16)};
 }
 
 enum { BAND_VF = 0, BAND_VFT = 1, BAND_VVT = 2 };

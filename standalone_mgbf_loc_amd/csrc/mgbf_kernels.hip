@@ -134,10 +134,13 @@ vband_kernel(const float* __restrict__ in, float* __restrict__ out,
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
 constexpr int kVColMaxHB = 8;     // hz <= 8 for Vf and Vf^T, <= 4 for their product
-// Shorter columns give a block too few values beside its two waits: 1024 x 1024
-// points at HB = 1, 5 levels in 20 us against 13 with the block above, 7 in 22
-// against 18; at HB = 3, 11 in 27.8 against 27.1 and 13 in 29 against 31
-constexpr int kVColMinLm = 13;
+// Shorter columns give a block too few values beside its two waits, which tells
+// on large fields: 1024 x 1024 points at HB = 1, 5 levels in 20 us against 13 with
+// the block above, 7 in 22 against 18; at HB = 3, 9 in 26 against 23 and 11 in 27.8
+// against 27.1. On small ones its launch is the shorter: 256 x 256 x 5 in 4.1 us
+// against 5.5, even at 512 x 512 (7.5 against 7.0; 7 levels 8.1 against 7.9).
+constexpr int kVColMinLm = 11;
+constexpr long long kVColSmall = 1 << 18;   // columns
 constexpr int kVColMaxLm = 128;   // 32 KB of columns: 4 blocks, 16 waves a CU
 constexpr int kVColWaves = kBlock / kWave;
 constexpr int kVColStep = 8;      // levels between shifts of the window
@@ -610,7 +613,7 @@ hipError_t launch_vband_h(const VBandArgs& a, hipStream_t st) {
     const long long N = (long long)a.K * a.npts;
     // whole columns of a length that spreads them over the LDS banks
     const long long ncol = a.nfilt == a.K && a.K % a.lm == 0 ? N / a.lm : 0;
-    if constexpr (HB <= kVColMaxHB) if (!fixl && ncol && a.lm % 4 && a.lm >= kVColMinLm && a.lm <= kVColMaxLm && ncol <= (1ll << 30) - kWave) {   // 4 threads a column, below 2^32
+    if constexpr (HB <= kVColMaxHB) if (!fixl && ncol && a.lm % 4 && (a.lm >= kVColMinLm || ncol < kVColSmall) && a.lm <= kVColMaxLm && ncol <= (1ll << 30) - kWave) {   // 4 threads a column, below 2^32
         const dim3 g((unsigned)((ncol + kWave - 1) / kWave));
         const size_t lds = sizeof(float) * kWave * (a.lm + kVColWaves * HB);
         // 64 columns start at a multiple of 256 bytes from the base

@@ -46,10 +46,3 @@ def test_default_heights_of_narrow_filters(n, lm, n_ens, h, kw):
         for tj in (48, 96):
             op.set_tiles({k: (4, min(tj, v[1]) if k[0] > 1 else tj) for k, v in tiles.items()})
             assert default <= 1.15 * _time(op, x, y), tj
-
-
-def test_plain_pass_of_a_small_field_has_short_tiles():
-    # 48 waves a row of tiles: 16 rows give 2880 waves, the 23 of one round of
-    # 2048 waves take 1.16 to 1.18 times as long
-    with M.MGBF(M.Config.for_grid(192, 960, 32, n_ens=2, gm=3, h=3, hz=2)) as op:
-        assert op.tiles()[(1, 0)][1] <= 16
