@@ -1,5 +1,5 @@
 """Vertical bands over columns that fit no power of two (whole columns in LDS
-from 13 to 128 levels, 4 not dividing them; a value a thread else) against the
+to 128 levels that 4 does not divide; a value a thread else) against the
 FP64 oracle: Vf and Vf^T at each half-width, on aligned and unaligned fields,
 and their product, of twice the half-width, at the end of W A W^T with constant
 weights. Normwise relative errors as in test_gpu_parity.py: 2e-6 for stages,
